@@ -23,18 +23,36 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
   return __uint_as_float(static_cast<uint32_t>(h) << 16);
 }
 
-// fp32 -> bf16, round to nearest even (NaN kept quiet), as torch's .to(bfloat16).
-// Written as a select, not an early return: the compiler turns the early
-// return into a divergent branch per value (~15 exec-mask instructions), which
-// made the GEMM epilogues several times longer than their arithmetic.
+// fp32 -> bf16, round to nearest even (NaN kept quiet), as torch's
+// .to(bfloat16), by gfx950's own conversion (v_cvt_pk_bf16_f32: equal to the
+// integer form ((u + 0x7fff + lsb) >> 16, NaN quieted) on all 2^32 inputs).
+// One instruction for two values instead of ~6 each.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
+}
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-  const uint32_t u = __float_as_uint(f);
-  const uint32_t rne = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-  const uint32_t qnan = (u >> 16) | 0x40u;
-  return static_cast<uint16_t>((u & 0x7fffffffu) > 0x7f800000u ? qnan : rne);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
+// both values rounded to bf16, back in fp32
+__device__ __forceinline__ void round_bf16x2(float& a, float& b) {
+  const uint32_t w = pack_bf16x2(a, b);
+  a = __uint_as_float(w << 16);
+  b = __uint_as_float(w & 0xffff0000u);
+}
+
+// n / d for d >= 1 (the sigmoid denominators): reciprocal, one residual step,
+// and the hardware's fix-up for infinities and NaN.  The general division's
+// operand scaling guards denormal operands and quotients that this
+// denominator does not have, at twice the instructions (11 against 5).
+__device__ __forceinline__ float div_ge1(float n, float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q = n * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, n), r, q), d, n);
+}
 
 // v / s correctly rounded (as a plain division, s > 0), then clamped to the
 // e4m3 range: v * (1/s) plus one FMA-residual correction (inv = 1/s, itself
@@ -60,7 +78,7 @@ __device__ __forceinline__ uint32_t pack_e4m3x4(float a, float b, float c, float
 
 __device__ __forceinline__ float silu_mul(float g, float u) {
   // ops/fused_moe.py:46 — gate / (1 + exp(-gate)) * up, in fp32
-  return (g / (1.0f + __expf(-g))) * u;
+  return div_ge1(g, 1.0f + __expf(-g)) * u;
 }
 
 // ------------------------------------------------------------- wave utils

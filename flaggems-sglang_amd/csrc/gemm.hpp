@@ -96,9 +96,10 @@ __device__ __forceinline__ float gemm1_act(const GemmParams& p, float ga, float 
       gv = fminf(gv, p.limit);
       lv = fminf(fmaxf(lv, -p.limit), p.limit);
     }
-    return gv / (1.0f + __expf(-p.alpha * gv)) * (lv + 1.0f) * g;
+    return div_ge1(gv, 1.0f + __expf(-p.alpha * gv)) * (lv + 1.0f) * g;
   } else {
-    const float gv = round_bf16(ga * g), uv = round_bf16(ua * g);
+    float gv = ga * g, uv = ua * g;
+    round_bf16x2(gv, uv);
     if constexpr (ACT == kActGelu) return 0.5f * gv * (1.0f + erff(gv * 0.7071067811865476f)) * uv;
     return silu_mul(gv, uv);
   }

@@ -72,6 +72,9 @@ struct Cfg {
   // waves, which carry the fewer units when the split is uneven
   static constexpr int SA_WAVES = FP8 ? (BM + 63) / 64 : 0;
   static constexpr int SA_FIRST = NW - SA_WAVES;
+  // 16-row weight blocks taken in pairs (see tile_col): a lane's results of a
+  // pair are 8 consecutive output columns
+  static constexpr bool PAIR = (MODE == Mode::kGemm1Silu ? NI / 2 : NI) % 2 == 0;
   // fp8 weight-scale stages held in LDS (the reduction dim is at most 128 KST)
   static constexpr int KST =
       NBUF * STAGE + NBUF * BM * 4 + WAVES_N * 2 * kMaxKStages * 4 <= 160 * 1024 ? kMaxKStages : 64;
@@ -150,36 +153,27 @@ __device__ __forceinline__ int find_expert(const int32_t* offs_pad, int E, int k
   return base + (63 - __builtin_clzll(b));
 }
 
-// 4x4 transpose across each quad of lanes (q = lane % 4): on entry v[r] of
-// lane q is element (column q, row r), on exit v[c] is element (column c,
-// row q).  Two exchange steps (lane bit 0 with element bit 0, then bit 1),
-// each two DPP quad permutes.
-template <int CTRL>
-__device__ __forceinline__ float qperm(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+// Which weight row of a tile sits in row lr of its 16-row LDS block b.  The
+// MFMA takes the weight fragment as its first operand, so a lane ends with
+// four consecutive weight rows 4 * (lane / 16) + 0..3 (output columns) of one
+// slot row, lane % 16: what a row store wants, with no exchange between lanes.
+// With PAIR, the rows of blocks 2p and 2p + 1 are dealt out four by four, so
+// a lane's two blocks are 8 consecutive columns (one 16-byte bf16 store, and
+// 64 contiguous bytes per row and instruction).  fp8: one activation scale
+// per lane and row block instead of four.  Against the opposite operand order
+// with 4x4 lane transposes and integer bf16 rounding in the epilogue, outputs
+// bit-identical: Mixtral bf16 M=4096 2707 -> 2626 us a call, Qwen3 M=8192
+// 891 -> 817 us, reference sweep M=1024 436 -> 416 us, DSV3 fp8 M=4096
+// 2991 -> 2724 us.
+template <bool PAIR>
+__device__ __forceinline__ int tile_row(int b, int lr) {
+  if constexpr (PAIR) return (b >> 1) * 32 + (lr >> 2) * 8 + (b & 1) * 4 + (lr & 3);
+  return b * 16 + lr;
 }
-__device__ __forceinline__ void quad_transpose(f32x4_t& v, int lane) {
-  const bool p0 = lane & 1, p1 = lane & 2;
-  float s0 = p0 ? v[0] : v[1], s1 = p0 ? v[2] : v[3];
-  float r0 = qperm<0xB1>(s0), r1 = qperm<0xB1>(s1);  // quad_perm [1,0,3,2]
-  if (p0) {
-    v[0] = r0;
-    v[2] = r1;
-  } else {
-    v[1] = r0;
-    v[3] = r1;
-  }
-  s0 = p1 ? v[0] : v[2];
-  s1 = p1 ? v[1] : v[3];
-  r0 = qperm<0x4E>(s0);  // quad_perm [2,3,0,1]
-  r1 = qperm<0x4E>(s1);
-  if (p1) {
-    v[0] = r0;
-    v[1] = r1;
-  } else {
-    v[2] = r0;
-    v[3] = r1;
-  }
+// First of the lane's four output columns of block j (same numbering).
+template <bool PAIR>
+__device__ __forceinline__ int tile_col(int j, int lane) {
+  return tile_row<PAIR>(j, (lane >> 4) * 4);
 }
 
 // Logical tile L (within one split) -> expert, N-tile and rows.  Per expert,
@@ -309,8 +303,8 @@ __global__ __launch_bounds__(256) void tail_fold_kernel(GemmParams p, int stages
     const int idx = (threadIdx.x + v * 256) * 4;
     const int r = idx / BN, c = idx - (idx / BN) * BN;
     if (r0 + r >= re - rb || c >= cols) continue;
-    const uint32_t w0 = f32_to_bf16(a[v].x) | (static_cast<uint32_t>(f32_to_bf16(a[v].y)) << 16);
-    const uint32_t w1 = f32_to_bf16(a[v].z) | (static_cast<uint32_t>(f32_to_bf16(a[v].w)) << 16);
+    const uint32_t w0 = pack_bf16x2(a[v].x, a[v].y);
+    const uint32_t w1 = pack_bf16x2(a[v].z, a[v].w);
     *reinterpret_cast<uint2*>(y + static_cast<int64_t>(rb + r0 + r) * p.Nout + c0 + c) = make_uint2(w0, w1);
   }
 }
@@ -419,7 +413,7 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     if (u < C::A_UNITS) {
       src[i] = p.A + a_src_row(b * 16 + lr) * kbytes + static_cast<int64_t>(k0) * SB + coff;
     } else {
-      const int r = (b - BM / 16) * 16 + lr;  // row of the B tile
+      const int r = tile_row<C::PAIR>(b - BM / 16, lr);  // row of the B tile
       int64_t brow;
       if (MODE == Mode::kGemm1Silu) {
         const int w = r / WN, within = r % WN;
@@ -491,16 +485,15 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
       const float* sa_st = sa_lds[kt % NBUF];
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        float sa[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sa[r] = sa_st[wm * WM + i * 16 + (lane >> 4) * 4 + r];
+        const float sa = sa_st[wm * WM + i * 16 + (lane & 15)];
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
           f32x4_t t = {0.f, 0.f, 0.f, 0.f};
-          t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[i], fb[j], t, 0, 0, 0, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[j], fa[i], t, 0, 0, 0, 0, 0, 0);
           const float sb = (MODE == Mode::kGemm1Silu ? j >= NI / 2 : j >= sb_split) ? sb1 : sb0;
+          const float sab = sa * sb;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] += t[r] * (sa[r] * sb);
+          for (int r = 0; r < 4; ++r) acc[i][j][r] += t[r] * sab;
         }
       }
     } else {
@@ -525,7 +518,7 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
         for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int j = 0; j < NI; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[h][i], fb[h][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[h][j], fa[h][i], acc[i][j], 0, 0, 0);
       if constexpr (UPB == 2) {
         // schedule: the first k-step's reads, then the second k-step's reads
         // spread over the first k-step's MFMAs, then the remaining MFMAs
@@ -589,13 +582,9 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     if (wave_live) compute(kt);
   }
 
-  // ---- epilogue.  C layout of a 16x16 block: lane holds column lane%16,
-  // rows 4*(lane/16) + r.  A 4x4 transpose inside each quad of lanes turns
-  // that into row 4*(lane/16) + lane%4, columns 4*((lane/4)%4) + 0..3, so each
-  // lane stores 4 consecutive outputs at once (8 or 16 bytes) instead of 4
-  // scattered ones.
-  const int orow = (lane >> 4) * 4 + (lane & 3);   // row within the 16x16 block
-  const int ocol = ((lane >> 2) & 3) * 4;          // first of the lane's 4 columns
+  // ---- epilogue.  The lane holds slot row lane % 16 of each 16-row block i
+  // and output columns tile_col(j, lane) + 0..3 of each weight block j.
+  const int orow = lane & 15;
   // Routing weights of the lane's rows, loaded and waited for before the
   // first store.  On gfx9 loads and stores share the vmcnt counter and the
   // compiler treats them as completing out of order, so a use of a load that
@@ -615,7 +604,7 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   if (MODE == Mode::kGemm2 && p.bias && split == 0) {
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
-      const int64_t col = static_cast<int64_t>(nt) * BN + wn * WN + j * 16 + ocol;
+      const int64_t col = static_cast<int64_t>(nt) * BN + wn * WN + tile_col<C::PAIR>(j, lane);
       if (col < p.Nout) {
         const float* b = p.bias + static_cast<int64_t>(e) * p.Nout + col;
 #pragma unroll
@@ -631,7 +620,7 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     if (p.act_q) {
       // Activation quantized here, exactly as fmoe_quant_fp8_group would do
       // it on the bf16 activation: the tile's 128 activation columns are one
-      // 1x128 group of each row.  Row amax: the lane's 8 values, the 4 lanes
+      // 1x128 group of each row.  Row amax: the lane's values, the 4 lanes
       // holding the row's other columns of this wave, then the WAVES_N waves
       // through LDS (the operand ring is free once every wave has left the
       // main loop).
@@ -644,21 +633,21 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
         float amax = 0.f;
 #pragma unroll
         for (int j = 0; j < NI / 2; ++j) {
-          f32x4_t gv = acc[i][j], uv = acc[i][j + NI / 2];
-          quad_transpose(gv, lane);
-          quad_transpose(uv, lane);
-          const int64_t col = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2) + j * 16 + ocol;
+          const int64_t col = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2) + tile_col<C::PAIR>(j, lane);
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             float gb, ub;
             gemm1_bias<ACT>(p, e, col + c, gb, ub);
-            v[i][j][c] = round_bf16(gemm1_act<ACT>(p, gv[c], uv[c], gb, ub, g));
-            amax = fmaxf(amax, fabsf(v[i][j][c]));
+            v[i][j][c] = gemm1_act<ACT>(p, acc[i][j][c], acc[i][j + NI / 2][c], gb, ub, g);
           }
+          round_bf16x2(v[i][j][0], v[i][j][1]);
+          round_bf16x2(v[i][j][2], v[i][j][3]);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) amax = fmaxf(amax, fabsf(v[i][j][c]));
         }
-        amax = fmaxf(amax, __shfl_xor(amax, 4, kWave));
-        amax = fmaxf(amax, __shfl_xor(amax, 8, kWave));
-        if (((lane >> 2) & 3) == 0) amax_lds[(wm * WM + i * 16 + orow) * C::WAVES_N + wn] = amax;
+        amax = fmaxf(amax, __shfl_xor(amax, 16, kWave));
+        amax = fmaxf(amax, __shfl_xor(amax, 32, kWave));
+        if (lane < 16) amax_lds[(wm * WM + i * 16 + orow) * C::WAVES_N + wn] = amax;
       }
       __syncthreads();
       const int64_t ngrp = p.N_act / 128;
@@ -672,20 +661,35 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
         const float sc = fmaxf(amax, kFp8Eps) / kFp8Max;
         const float inv = 1.0f / sc;
         if (s >= row_end) continue;
-        uint8_t* q = p.act_q + static_cast<int64_t>(s) * p.N_act;
+        uint8_t* q = p.act_q + static_cast<int64_t>(s) * p.N_act + static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2);
+        uint32_t w[NI / 2];
 #pragma unroll
-        for (int j = 0; j < NI / 2; ++j) {
-          const int64_t col = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2) + j * 16 + ocol;
-          *reinterpret_cast<uint32_t*>(q + col) =
-              pack_e4m3x4(fp8_qdiv(v[i][j][0], sc, inv), fp8_qdiv(v[i][j][1], sc, inv),
-                          fp8_qdiv(v[i][j][2], sc, inv), fp8_qdiv(v[i][j][3], sc, inv));
+        for (int j = 0; j < NI / 2; ++j)
+          w[j] = pack_e4m3x4(fp8_qdiv(v[i][j][0], sc, inv), fp8_qdiv(v[i][j][1], sc, inv),
+                             fp8_qdiv(v[i][j][2], sc, inv), fp8_qdiv(v[i][j][3], sc, inv));
+        if constexpr (C::PAIR) {
+#pragma unroll
+          for (int j = 0; j < NI / 2; j += 2)
+            *reinterpret_cast<uint2*>(q + tile_col<true>(j, lane)) = make_uint2(w[j], w[j + 1]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < NI / 2; ++j) *reinterpret_cast<uint32_t*>(q + tile_col<false>(j, lane)) = w[j];
         }
-        if (wn == 0 && ((lane >> 2) & 3) == 0) p.act_qs[static_cast<int64_t>(s) * ngrp + nt] = sc;
+        if (wn == 0 && lane < 16) p.act_qs[static_cast<int64_t>(s) * ngrp + nt] = sc;
       }
       return;
     }
   }
   const bool y_rows_bf16 = p.y_bf16 && tail < 0;  // whole tile, one split: bf16 slot rows
+  // four bf16 columns of blocks j (and j + 1) of a row: one 16- or 8-byte store
+  auto store_bf16 = [&](uint16_t* row, int64_t c0, int j, const uint32_t* w) {
+    uint16_t* dst = row + c0 + tile_col<C::PAIR>(j, lane);
+    if constexpr (C::PAIR)
+      *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+    else
+      *reinterpret_cast<uint2*>(dst) = make_uint2(w[0], w[1]);
+  };
+  constexpr int JS = C::PAIR ? 2 : 1;  // blocks per store
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int s = row_beg + wm * WM + i * 16 + orow;
@@ -693,25 +697,24 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     const float g = gv[i];
     if (MODE == Mode::kGemm1Silu) {
       uint16_t* act = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(s) * p.N_act;
+      const int64_t c0 = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2);
 #pragma unroll
-      for (int j = 0; j < NI / 2; ++j) {
-        f32x4_t gv = acc[i][j], uv = acc[i][j + NI / 2];
-        quad_transpose(gv, lane);
-        quad_transpose(uv, lane);
-        uint32_t w[2];
-        const int64_t col = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2) + j * 16 + ocol;
+      for (int j = 0; j < NI / 2; j += JS) {
+        uint32_t w[2 * JS];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int h = 0; h < 2 * JS; ++h) {
+          const int jj = j + h / 2, c = 2 * (h % 2);
+          const int64_t col = c0 + tile_col<C::PAIR>(jj, lane) + c;
           float a[2];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
+          for (int u = 0; u < 2; ++u) {
             float gb, ub;
-            gemm1_bias<ACT>(p, e, col + 2 * c + h, gb, ub);
-            a[h] = gemm1_act<ACT>(p, gv[2 * c + h], uv[2 * c + h], gb, ub, g);
+            gemm1_bias<ACT>(p, e, col + u, gb, ub);
+            a[u] = gemm1_act<ACT>(p, acc[i][jj][c + u], acc[i][jj + NI / 2][c + u], gb, ub, g);
           }
-          w[c] = f32_to_bf16(a[0]) | (static_cast<uint32_t>(f32_to_bf16(a[1])) << 16);
+          w[h] = pack_bf16x2(a[0], a[1]);
         }
-        if (ok && col < p.N_act) *reinterpret_cast<uint2*>(act + col) = make_uint2(w[0], w[1]);
+        if (ok && c0 + tile_col<C::PAIR>(j, lane) < p.N_act) store_bf16(act, c0, j, w);
       }
     } else {
       // fp32 destination row: a split plane's slot row, or the tile's row of
@@ -722,25 +725,34 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
                                  (wm * WM + i * 16 + orow) * BN - static_cast<int64_t>(nt) * BN
                            : static_cast<float*>(p.out) + split * p.out_split_stride +
                                  static_cast<int64_t>(s) * p.Nout;
+      uint16_t* yb = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(s) * p.Nout;
+      const int64_t c0 = static_cast<int64_t>(nt) * BN + wn * WN;
 #pragma unroll
-      for (int j = 0; j < NI; ++j) {
-        f32x4_t v = acc[i][j];
-        quad_transpose(v, lane);
-        const int64_t col = static_cast<int64_t>(nt) * BN + wn * WN + j * 16 + ocol;
-        if (p.bias && split == 0) {
+      for (int j = 0; j < NI; j += JS) {
+        f32x4_t v[JS];
 #pragma unroll
-          for (int c = 0; c < 4; ++c) v[c] += bv[j][c];
+        for (int h = 0; h < JS; ++h) {
+          v[h] = acc[i][j + h];
+          if (p.bias && split == 0) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[h][c] += bv[j + h][c];
+          }
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[h][c] *= g;
         }
+        const int64_t col = c0 + tile_col<C::PAIR>(j, lane);
         if (ok && col < p.Nout) {
           if (y_rows_bf16) {
             // one split: the row goes out as bf16, like SGLang's per-slot
             // intermediate before its top-k sum
-            uint16_t* yb = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(s) * p.Nout + col;
-            const uint32_t w0 = f32_to_bf16(v[0] * g) | (static_cast<uint32_t>(f32_to_bf16(v[1] * g)) << 16);
-            const uint32_t w1 = f32_to_bf16(v[2] * g) | (static_cast<uint32_t>(f32_to_bf16(v[3] * g)) << 16);
-            *reinterpret_cast<uint2*>(yb) = make_uint2(w0, w1);
+            uint32_t w[2 * JS];
+#pragma unroll
+            for (int h = 0; h < 2 * JS; ++h) w[h] = pack_bf16x2(v[h / 2][2 * (h % 2)], v[h / 2][2 * (h % 2) + 1]);
+            store_bf16(yb, c0, j, w);
           } else {
-            *reinterpret_cast<float4*>(y + col) = make_float4(v[0] * g, v[1] * g, v[2] * g, v[3] * g);
+#pragma unroll
+            for (int h = 0; h < JS; ++h)
+              *reinterpret_cast<float4*>(y + col + 4 * h) = make_float4(v[h][0], v[h][1], v[h][2], v[h][3]);
           }
         }
       }

@@ -122,8 +122,8 @@ __global__ __launch_bounds__(kSumThreads) void moe_sum_kernel(const YT* __restri
           acc[3] += v[u][3];
         }
     }
-    const uint32_t w0 = f32_to_bf16(acc[0] * scale) | (static_cast<uint32_t>(f32_to_bf16(acc[1] * scale)) << 16);
-    const uint32_t w1 = f32_to_bf16(acc[2] * scale) | (static_cast<uint32_t>(f32_to_bf16(acc[3] * scale)) << 16);
+    const uint32_t w0 = pack_bf16x2(acc[0] * scale, acc[1] * scale);
+    const uint32_t w1 = pack_bf16x2(acc[2] * scale, acc[3] * scale);
     *reinterpret_cast<uint2*>(out + t * K + c) = make_uint2(w0, w1);
   }
 }
@@ -185,8 +185,7 @@ __global__ __launch_bounds__(256) void moe_sum_rows_bf16_kernel(const uint16_t* 
       i32x4_t o;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        o[q] = static_cast<int>(f32_to_bf16(acc[h][2 * q] * scale) |
-                                (static_cast<uint32_t>(f32_to_bf16(acc[h][2 * q + 1] * scale)) << 16));
+        o[q] = static_cast<int>(pack_bf16x2(acc[h][2 * q] * scale, acc[h][2 * q + 1] * scale));
       *reinterpret_cast<i32x4_t*>(out + t * K + (c0 + h * kWave) * 8) = o;
     }
   }
@@ -300,8 +299,8 @@ __global__ __launch_bounds__(256) void moe_sum_planes_kernel(const float* __rest
     sum.z += v.z;
     sum.w += v.w;
   }
-  const uint32_t w0 = f32_to_bf16(sum.x * scale) | (static_cast<uint32_t>(f32_to_bf16(sum.y * scale)) << 16);
-  const uint32_t w1 = f32_to_bf16(sum.z * scale) | (static_cast<uint32_t>(f32_to_bf16(sum.w * scale)) << 16);
+  const uint32_t w0 = pack_bf16x2(sum.x * scale, sum.y * scale);
+  const uint32_t w1 = pack_bf16x2(sum.z * scale, sum.w * scale);
   *reinterpret_cast<uint2*>(out + t * K + c) = make_uint2(w0, w1);
 }
 

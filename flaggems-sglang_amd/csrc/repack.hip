@@ -199,7 +199,7 @@ __global__ __launch_bounds__(kThreads) void dequant_4bit_kernel(const uint8_t* _
     for (int b = 0; b < 4; ++b) {
       const float lo = (static_cast<float>((word >> (8 * b)) & 15u) - z) * s;
       const float hi = (static_cast<float>((word >> (8 * b + 4)) & 15u) - z) * s;
-      w[b] = f32_to_bf16(lo) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
+      w[b] = pack_bf16x2(lo, hi);
     }
   }
   *reinterpret_cast<i32x4_t*>(out + row * K + 8 * m) =
