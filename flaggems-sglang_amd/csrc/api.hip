@@ -73,6 +73,17 @@ int check_routing(const fmoe_routing* r, const char* who) {
 // Decode (block_m 16) or prefill (64 / 128) kernels follow the routing's tile height.
 bool is_decode(const fmoe_routing* r) { return r->block_m == kDecodeBM; }
 
+// Most tiles of height bm that `slots` slots over E experts make: every expert
+// that has slots may end in a partial tile.  fmoe_max_tiles bounds any tile
+// height (it sizes tile_map); the prefill grids take this one, because every
+// workgroup past the live tiles still waits for a CU's whole LDS before it
+// can leave (Mixtral M=4096: 519 tiles against 40, 54,000 empty workgroups in
+// the GEMM1 launch).
+int64_t prefill_max_tiles(int64_t slots, int64_t E, int bm) {
+  const int64_t used = slots < E ? slots : E;  // experts with slots
+  return (slots + used * (bm - 1)) / bm;
+}
+
 GemmParams base_params(const fmoe_routing* r) {
   GemmParams p{};
   p.topk_indx = r->topk_indx;
@@ -84,6 +95,10 @@ GemmParams base_params(const fmoe_routing* r) {
   p.top_k = r->top_k;
   p.n_experts = r->n_experts;
   p.max_tiles = r->max_tiles;
+  if (!is_decode(r)) {
+    const int64_t t = prefill_max_tiles(r->n_tokens * r->top_k, r->n_experts, r->block_m);
+    if (t < p.max_tiles) p.max_tiles = static_cast<int>(t);
+  }
   p.splits = 1;
   p.act = FMOE_ACT_SILU;
   p.bias = nullptr;
@@ -417,7 +432,7 @@ FusedLayout layout(const fmoe_fused_args* a) {
   // slots: Qwen3 M=8192 GEMM2 351 -> 387 us, DSV3 M=4096 1107 -> 1158 us).
   L.tail_bytes = (L.bm != kDecodeBM && !L.fused4 && L.splits > 1 &&
                   (a->wtype == FMOE_W_BF16 || a->wtype == FMOE_W_FP8))
-                     ? prefill_tail_bytes(to_wt(a->wtype), L.bm, L.max_tiles, a->K)
+                     ? prefill_tail_bytes(to_wt(a->wtype), L.bm, prefill_max_tiles(slots, a->E, L.bm), a->K)
                      : 0;
   if (L.tail_bytes > 0) L.splits = 1;
   size_t off = 0;
@@ -449,7 +464,8 @@ FusedLayout layout(const fmoe_fused_args* a) {
   // prefill: logical-tile table, shared by the two GEMM launches (stream order)
   const int64_t nn1 = (a->N + kPrefillBN / 2 - 1) / (kPrefillBN / 2);
   const int64_t nn2 = (a->K + kPrefillBN - 1) / kPrefillBN;
-  L.lut = take(L.bm == kDecodeBM ? 0 : 16 * static_cast<size_t>(L.max_tiles) * (nn1 > nn2 ? nn1 : nn2));
+  L.lut = take(L.bm == kDecodeBM ? 0
+                                 : 16 * static_cast<size_t>(prefill_max_tiles(slots, a->E, L.bm)) * (nn1 > nn2 ? nn1 : nn2));
   L.tail = take(L.tail_bytes);
   L.total = off;
   return L;
