@@ -38,6 +38,7 @@
 // tail_fold_kernel adds; the top-k sum runs in its own fixed-order launch
 // (deterministic).
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm.hpp"
 
@@ -93,12 +94,15 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4) | (0xf << 8));
 }
 
-// wait until at most `newer` stages (P loads each) of this wave are in flight
-template <int P>
-__device__ __forceinline__ void wait_ring(int newer) {
-  if (newer >= 2) wait_vmcnt<2 * P>();
-  else if (newer == 1) wait_vmcnt<P>();
-  else wait_vmcnt<0>();
+// wait until at most n of this wave's loads are in flight (n uniform, 0..MAX)
+template <int MAX>
+__device__ __forceinline__ void wait_loads(int n) {
+  if constexpr (MAX == 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (n >= MAX) wait_vmcnt<MAX>();
+    else wait_loads<MAX - 1>(n);
+  }
 }
 
 __device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" ::: "memory"); }
@@ -371,12 +375,15 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     row_end = t.row_end;
   }
 
-  // GEMM2: waves whose rows are all padding skip their fragment reads and
-  // MFMAs.  An expert's last M-tile is often nearly empty (Mixtral M=4096:
-  // ~1024 +- 30 slots per expert, so about half the experts add a fifth
-  // 256-row tile of a few dozen rows).  Measured: GEMM2 -0.5 to -1.5% on the
-  // BASELINE prefill shapes; GEMM1 +2-3% with the same skip, so not there.
-  const bool wave_live = C::WAVES_M == 1 || MODE == Mode::kGemm1Silu ||
+  // An expert's last M-tile is often nearly empty (Mixtral M=4096: ~1024 +- 30
+  // slots per expert, so about half the experts add a fifth 256-row tile of a
+  // few dozen rows; Qwen3 M=8192: a fifth of all tile rows are padding).
+  // Waves whose rows are all padding skip their fragment reads and MFMAs, and
+  // bf16 tiles do not fetch the DMA units of padding rows (their LDS rows hold
+  // whatever was there; a slot row's results depend on its own operand row
+  // only).  fp8 GEMM1 does neither (its 160-row tiles are mostly full: DSV3
+  // M=4096 +3% with both).
+  const bool wave_live = C::WAVES_M == 1 || (FP8 && MODE == Mode::kGemm1Silu) ||
                          __builtin_amdgcn_readfirstlane(row_end - row_beg > wm * WM);
 
   const int ksb = static_cast<int>(p.Kred / 128);      // fp8 scale blocks per row
@@ -395,7 +402,16 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   const uint8_t* Be = p.B + static_cast<int64_t>(e) * p.Nout * kbytes;
   const uint8_t* src[C::UPW];
   int loff[C::UPW];
-  const bool full_wave = C::REM == 0 || wid < C::REM;  // issues UPW units (else UPW - 1)
+  // the units this wave issues: UPW or UPW - 1, less those of padding rows
+  uint32_t units = C::REM == 0 || wid < C::REM ? (1u << C::UPW) - 1 : (1u << (C::UPW - 1)) - 1;
+  if constexpr (!FP8) {
+#pragma unroll
+    for (int i = 0; i < C::UPW; ++i) {
+      const int u = NW * i + wid;
+      if (u < C::A_UNITS && u * (16 / UPB) >= row_end - row_beg) units &= ~(1u << i);
+    }
+  }
+  units = __builtin_amdgcn_readfirstlane(units);
 #pragma unroll
   for (int i = 0; i < C::UPW; ++i) {
     const int u = min(NW * i + wid, C::UNITS - 1);
@@ -435,12 +451,13 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   const float* sa_src = nullptr;
   if (sa_wave) sa_src = p.a_scale + a_src_row(min(64 * sa_j + lane, BM - 1)) * ksb + k0;
   int sb_split = NI;  // GEMM2: 16-row blocks of the wave under its first weight-scale block
+  // unit i of stage kt
+  auto issue_unit = [&](int kt, int i) {
+    if ((FP8 && i + 1 < C::UPW) || (units >> i & 1)) dma16(src[i] + static_cast<int64_t>(kt) * SB, lds[kt % NBUF] + loff[i]);
+  };
   auto issue = [&](int kt) {
-    uint8_t* st = lds[kt % NBUF];
-    const int64_t off = static_cast<int64_t>(kt) * SB;
 #pragma unroll
-    for (int i = 0; i < C::UPW; ++i)
-      if (i + 1 < C::UPW || full_wave) dma16(src[i] + off, st + loff[i]);
+    for (int i = 0; i < C::UPW; ++i) issue_unit(kt, i);
     if (sa_wave) {
       if (64 * (sa_j + 1) <= BM) {
         dma4(sa_src + kt, &sa_lds[kt % NBUF][64 * sa_j]);
@@ -459,17 +476,68 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   // per-lane fragment offsets within a 16-row block's units
   const int foff0 = frag_off<SB>(lane, lane >> 4);
   const int foff1 = SB == 64 ? 0 : frag_off<SB>(lane, 4 + (lane >> 4));
-  // The wave raises its issue priority for its fragment reads and MFMAs and
-  // drops it before the next stage's wait and DMA issue: bf16 (Mixtral
-  // M=4096 GEMM1 1.90 -> 1.86 ms, Qwen3 M=8192 GEMM1 -1%) and fp8 GEMM2
-  // (DSV3 M=4096 -1.3%); fp8 GEMM1 keeps one level (+3.6% with it)
-  constexpr int kPrio = (FP8 && MODE == Mode::kGemm1Silu) ? 0 : 1;
-  auto compute = [&](int kt) {
-    if (kPrio) __builtin_amdgcn_s_setprio(kPrio);
-    const uint8_t* st = lds[kt % NBUF];
-    const uint8_t* As = st + (wm * MI) * UPB * kUnit;
-    const uint8_t* Bs = st + (C::A_UNITS + wn * NI * UPB) * kUnit;
-    if constexpr (FP8) {
+  // DMA instructions per stage for this wave: its operand units, plus one
+  // a-scale load
+  const int per = __builtin_popcount(units) + (sa_wave ? 1 : 0);
+  // this wave's part of a stage has landed once at most `newer` younger stages
+  // are in flight; the whole stage after the barrier
+  auto wait_full = [&](auto newer) {  // a full ring: a constant count first
+    constexpr int N = decltype(newer)::value;
+    wait_loads<N * (C::UPW + (FP8 ? 1 : 0))>(N * per);
+    barrier_nofence();
+  };
+  auto wait_stage = [&](int newer) {
+    wait_loads<(NBUF - 1) * (C::UPW + (FP8 ? 1 : 0))>(newer * per);
+    barrier_nofence();
+  };
+  using Ring2 = std::integral_constant<int, NBUF - 2>;
+
+  if constexpr (FP8) {
+    // ring: up to NBUF-2 stages newer than kt stay in flight while kt is consumed
+#pragma unroll
+    for (int s = 0; s < NBUF - 1; ++s)
+      if (s < nk) issue(s);
+    // weight scales of the whole k range, staged once in LDS -- after the
+    // first stages' DMA is issued, so the two round trips overlap
+    const int64_t nrb = p.Nout / 128;
+    const float* se = p.b_scale + static_cast<int64_t>(e) * nrb * ksb;
+    const float* s0;
+    const float* s1;
+    if (MODE == Mode::kGemm1Silu) {
+      // the wave's gate rows (and up rows) lie in one 128-row scale block
+      const int64_t j = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2);
+      s0 = se + (gemm1_row(ACT, p.N_act, j, 0) / 128) * ksb;
+      s1 = se + (gemm1_row(ACT, p.N_act, j, 1) / 128) * ksb;
+    } else {
+      // the wave's rows span at most two 128-row scale blocks (WN <= 128):
+      // 16-row blocks j < sb_split use the first one
+      int64_t j = static_cast<int64_t>(nt) * BN + wn * WN;
+      if (j >= p.Nout) j = p.Nout - 1;
+      const int64_t jl = min(j + WN - 1, p.Nout - 1);
+      s0 = se + (j / 128) * ksb;
+      s1 = se + (jl / 128) * ksb;
+      if (jl / 128 != j / 128) sb_split = static_cast<int>((128 - j % 128) / 16);
+    }
+    if (wm == 0)
+      for (int kk = lane; kk < nk; kk += kWave) {
+        sb_lds[wn][0][kk] = s0[k0 + kk];
+        sb_lds[wn][1][kk] = s1[k0 + kk];
+      }
+    __syncthreads();
+    // GEMM2 raises the wave's issue priority for its fragment reads and MFMAs
+    // (DSV3 M=4096 -1.3%); GEMM1 keeps one level (+3.6% with it)
+    constexpr int kPrio = MODE == Mode::kGemm1Silu ? 0 : 1;
+    for (int kt = 0; kt < nk; ++kt) {
+      if (kt + NBUF - 1 < nk) {
+        wait_full(Ring2{});
+        issue(kt + NBUF - 1);
+      } else {
+        wait_stage(min(NBUF - 2, nk - 1 - kt));
+      }
+      if (!wave_live) continue;
+      if (kPrio) __builtin_amdgcn_s_setprio(kPrio);
+      const uint8_t* As = lds[kt % NBUF] + (wm * MI) * UPB * kUnit;
+      const uint8_t* Bs = lds[kt % NBUF] + (C::A_UNITS + wn * NI * UPB) * kUnit;
       i32x8_t fa[MI], fb[NI];
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
@@ -496,90 +564,111 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
           for (int r = 0; r < 4; ++r) acc[i][j][r] += t[r] * sab;
         }
       }
-    } else {
-      // every fragment of the stage is read up front, the second k-step's
-      // reads pinned between the first k-step's MFMAs (the scheduler would
-      // otherwise issue them after those MFMAs to save registers): Mixtral
-      // M=4096 GEMM1 1.95 -> 1.90 ms, GEMM2 1.06 -> 1.02 ms
-      bf16x8_t fa[UPB][MI], fb[UPB][NI];
+      if (kPrio) __builtin_amdgcn_s_setprio(0);
+    }
+  } else {
+    // bf16.  A step is 32 reduction elements: MI x NI MFMAs on fragments that
+    // were read from LDS during the step before, so the matrix cores do not
+    // wait for fragment reads.  Between a stage's last two steps its reads
+    // are over and the next stage's begin; there, one wait and one barrier
+    // both publish stage kt + 1 and free the slot of stage kt, whose DMA
+    // (stage kt + NBUF) goes out between that step's MFMAs.  Against reading
+    // a stage's first fragments after the barrier that publishes it and
+    // issuing the DMA in one go (and without the padding rows' share above),
+    // outputs bit-identical, same process: Mixtral M=4096 2614 -> 2530 us a
+    // call, Qwen3 M=8192 820 -> 779 us, reference sweep M=2048 622 -> 601 us.
+    // What bounds the 256 x 256 kernel now (Mixtral GEMM1 1750 us): with every
+    // operand line an L2 hit 1519 us, without the DMA 1353 us, without
+    // fragment reads as well 1230 us, the MFMAs alone 1.0 ms at 2.07 GHz.
+    constexpr int kMfma = MI * NI, NF = MI + NI;
+    constexpr int kRd = 2 * NF <= kMfma ? 2 : 1;  // MFMAs between fragment reads
+    // ... and between DMA units (2 / 3 / 4 measured at 256 x 256: Mixtral
+    // M=4096 2607 / 2562 / 2610 us a call; issued back to back they hold up
+    // the MFMAs, further apart they arrive late for a 2-deep ring)
+    constexpr int kDma = 3 * C::UPW <= kMfma ? 3 : (2 * C::UPW <= kMfma ? 2 : 1);
+    static_assert(NF <= kMfma && C::UPW <= kMfma, "reads and DMA fit between the MFMAs of a step");
+    bf16x8_t fa[2][MI], fb[2][NI];
+    // fragment f of step h of the stage in slot st, into register set q
+    auto read_frag = [&](const uint8_t* st, int h, int q, int f) {
+      const int fo = h == 0 ? foff0 : foff1;
+      if (f >= 1 && f <= NI)
+        fb[q][f - 1] = __builtin_bit_cast(bf16x8_t, lds16(st + (C::A_UNITS + (wn * NI + f - 1) * UPB) * kUnit + fo));
+      else
+        fa[q][f == 0 ? 0 : f - NI] =
+            __builtin_bit_cast(bf16x8_t, lds16(st + (wm * MI + (f == 0 ? 0 : f - NI)) * UPB * kUnit + fo));
+    };
+    // one step on register set q; READ: fragments of step h of slot st go to
+    // set 1 - q; DMA: stage kd goes out
+    auto step = [&](int q, auto rd, const uint8_t* st, int h, auto dm, int kd) {
+      constexpr bool READ = decltype(rd)::value, DMA = decltype(dm)::value;
 #pragma unroll
-      for (int h = 0; h < UPB; ++h) {
-        const int fo = h == 0 ? foff0 : foff1;
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-          fa[h][i] = __builtin_bit_cast(bf16x8_t, lds16(As + i * UPB * kUnit + fo));
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-          fb[h][j] = __builtin_bit_cast(bf16x8_t, lds16(Bs + j * UPB * kUnit + fo));
+      for (int m = 0; m < kMfma; ++m) {
+        const int i = m / NI, j = m % NI;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (READ)
+          if (m % kRd == 0 && m / kRd < NF) read_frag(st, h, 1 - q, m / kRd);
+        if constexpr (DMA)
+          if (m % kDma == 0 && m / kDma < C::UPW) issue_unit(kd, m / kDma);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[q][j], fa[q][i], acc[i][j], 0, 0, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    auto done_reading = [&] { __builtin_amdgcn_s_waitcnt(0xc07f); };  // lgkmcnt(0)
+
 #pragma unroll
-      for (int h = 0; h < UPB; ++h)
+    for (int s = 0; s < NBUF; ++s)
+      if (s < nk) issue(s);
+    wait_stage(min(NBUF - 1, nk - 1));
+    if (!wave_live) {
+      int kt = 0;
+      for (; kt + NBUF < nk; ++kt) {
+        wait_full(Ring2{});
+        issue(kt + NBUF);
+      }
+      for (; kt + 1 < nk; ++kt) wait_stage(min(NBUF - 2, nk - 2 - kt));
+    } else if (nk > 0) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[h][j], fa[h][i], acc[i][j], 0, 0, 0);
+      for (int f = 0; f < NF; ++f) read_frag(lds[0], 0, 0, f);
       if constexpr (UPB == 2) {
-        // schedule: the first k-step's reads, then the second k-step's reads
-        // spread over the first k-step's MFMAs, then the remaining MFMAs
-        constexpr int NF = MI + NI;  // fragment reads per k-step
-        __builtin_amdgcn_sched_group_barrier(0x100, NF, 0);
-#pragma unroll
-        for (int r = 0; r < NF; ++r) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        int kt = 0;
+        for (; kt + NBUF < nk; ++kt) {
+          step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
+          done_reading();
+          wait_full(Ring2{});
+          step(1, T{}, lds[(kt + 1) % NBUF], 0, T{}, kt + NBUF);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 2 * MI * NI - 2 * NF, 0);
+        for (; kt + 1 < nk; ++kt) {
+          step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
+          done_reading();
+          wait_stage(min(NBUF - 2, nk - 2 - kt));
+          step(1, T{}, lds[(kt + 1) % NBUF], 0, F{}, 0);
+        }
+        step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
+        step(1, F{}, nullptr, 0, F{}, 0);
+      } else {
+        // one step per stage: the register sets alternate with the stages
+        auto stage = [&](int kt, int q) {
+          if (kt + 1 < nk) {
+            done_reading();
+            if (kt + NBUF < nk) {
+              wait_full(Ring2{});
+              step(q, T{}, lds[(kt + 1) % NBUF], 0, T{}, kt + NBUF);
+            } else {
+              wait_stage(min(NBUF - 2, nk - 2 - kt));
+              step(q, T{}, lds[(kt + 1) % NBUF], 0, F{}, 0);
+            }
+          } else {
+            step(q, F{}, nullptr, 0, F{}, 0);
+          }
+        };
+        for (int kt = 0; kt < nk; kt += 2) {
+          stage(kt, 0);
+          if (kt + 1 < nk) stage(kt + 1, 1);
+        }
       }
     }
-    if (kPrio) __builtin_amdgcn_s_setprio(0);
-  };
-
-  // ring: up to NBUF-2 stages newer than kt stay in flight while kt is consumed
-#pragma unroll
-  for (int s = 0; s < NBUF - 1; ++s)
-    if (s < nk) issue(s);
-  // fp8 weight scales of the whole k range, staged once in LDS -- after the
-  // first stages' DMA is issued, so the two round trips overlap
-  if (FP8) {
-    const int64_t nrb = p.Nout / 128;
-    const float* se = p.b_scale + static_cast<int64_t>(e) * nrb * ksb;
-    const float* s0;
-    const float* s1;
-    if (MODE == Mode::kGemm1Silu) {
-      // the wave's gate rows (and up rows) lie in one 128-row scale block
-      const int64_t j = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2);
-      s0 = se + (gemm1_row(ACT, p.N_act, j, 0) / 128) * ksb;
-      s1 = se + (gemm1_row(ACT, p.N_act, j, 1) / 128) * ksb;
-    } else {
-      // the wave's rows span at most two 128-row scale blocks (WN <= 128):
-      // 16-row blocks j < sb_split use the first one
-      int64_t j = static_cast<int64_t>(nt) * BN + wn * WN;
-      if (j >= p.Nout) j = p.Nout - 1;
-      const int64_t jl = min(j + WN - 1, p.Nout - 1);
-      s0 = se + (j / 128) * ksb;
-      s1 = se + (jl / 128) * ksb;
-      if (jl / 128 != j / 128) sb_split = static_cast<int>((128 - j % 128) / 16);
-    }
-    if (wm == 0)
-      for (int kk = lane; kk < nk; kk += kWave) {
-        sb_lds[wn][0][kk] = s0[k0 + kk];
-        sb_lds[wn][1][kk] = s1[k0 + kk];
-      }
-    __syncthreads();
-  }
-
-  // DMA instructions per stage for this wave: UPW or UPW - 1 operand units,
-  // plus one a-scale load
-  const int per = (full_wave ? C::UPW : C::UPW - 1) + (sa_wave ? 1 : 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int newer = min(NBUF - 2, nk - 1 - kt);
-    if (per == C::UPW + 1) wait_ring<C::UPW + 1>(newer);
-    else if (per == C::UPW) wait_ring<C::UPW>(newer);
-    else wait_ring<(C::UPW > 1 ? C::UPW - 1 : 1)>(newer);
-    barrier_nofence();
-    if (kt + NBUF - 1 < nk) issue(kt + NBUF - 1);
-    if (wave_live) compute(kt);
   }
 
   // ---- epilogue.  The lane holds slot row lane % 16 of each 16-row block i

@@ -1,6 +1,7 @@
 """Prefill launches at the bound of their grid: routings in which every expert
 ends in a tile of one row make exactly (slots + E (block_m - 1)) / block_m
-tiles, the most that a batch can have, for each tile height."""
+tiles, the most that a batch can have, for each tile height -- over reduction
+lengths of 1 to 10 ring stages (fewer than the ring's depth, odd and even)."""
 
 import pytest
 import torch
@@ -10,7 +11,7 @@ from test_gpu_fused_moe import _close
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-K, N, E, k = 256, 384, 8, 2
+E, k = 8, 2
 
 COUNTS = {  # tile height -> slots per expert, each 1 modulo the height
     64: [65, 65] + [1] * 6,
@@ -26,9 +27,10 @@ def _ids(counts):
     return torch.stack((flat[:M], flat[M:]), dim=1).to(torch.int32)
 
 
+@pytest.mark.parametrize("K,N", [(128, 128), (256, 384), (384, 256), (640, 128), (128, 640)])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("bm", sorted(COUNTS))
-def test_every_expert_ends_in_a_one_row_tile(bm, fp8):
+def test_every_expert_ends_in_a_one_row_tile(bm, fp8, K, N):
     import flaggems_sglang
     from flaggems_sglang import _lib
     from flaggems_sglang import quant as Q
@@ -53,8 +55,8 @@ def test_every_expert_ends_in_a_one_row_tile(bm, fp8):
         # row by row, by norm: both sides round the activation to e4m3, and one
         # code flipped by another summation order moves an element by up to
         # 2^-3 of its largest term (seen: 0.11 rms on 1 of 1e5 elements), a row of
-        # N = 384 terms by 2^-3 / sqrt(384) = 0.6% of its norm per flip; a row from
-        # a missing or misplaced tile is off by its whole norm
+        # N terms by 2^-3 / sqrt(N) (N = 128: 1.1%) of its norm per flip;
+        # a row from a missing or misplaced tile is off by its whole norm
         err = (out.float().cpu() - ref.float()).norm(dim=1) / ref.float().norm(dim=1)
         assert float(err.max()) < 5e-2
     else:
