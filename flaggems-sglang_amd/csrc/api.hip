@@ -62,8 +62,8 @@ int check_routing(const fmoe_routing* r, const char* who) {
     return fail(FMOE_ERR_INVALID, "%s: routing pointer is null", who);
   if (r->n_tokens < 0 || r->top_k < 1 || r->n_experts < 1 || r->max_tiles < 0)
     return fail(FMOE_ERR_INVALID, "%s: bad routing sizes", who);
-  if (r->block_m != 16 && r->block_m != 64 && r->block_m != 128 && r->block_m != 160 &&
-      r->block_m != 256)
+  if (r->block_m != 16 && r->block_m != 32 && r->block_m != 64 && r->block_m != 128 &&
+      r->block_m != 160 && r->block_m != 256)
     return fail(FMOE_ERR_UNSUPPORTED, "%s: block_m=%d is not supported", who, r->block_m);
   if (r->block_m != 16 && !r->offs_pad)
     return fail(FMOE_ERR_INVALID, "%s: prefill routing needs offs_pad", who);
@@ -107,28 +107,54 @@ GemmParams base_params(const fmoe_routing* r) {
   return p;
 }
 
+// Slots per expert (of the experts that can have any) up to which the
+// streaming kernels run; above it the prefill kernels' LDS ring streams the
+// weights faster than the registers do (more bytes in flight per CU), decode
+// vs prefill kernels in us a call: bf16 Qwen3 M=128 (8 slots) 235 / 232, reference
+// sweep M=64 (8) 279 / 282, M=90 (11) 309 / 288 and M=128 (16) 374 / 294, Mixtral
+// M=40 (10) 497 / 506 and M=64 (16) 613 / 496; fp8 DSV3 M=64 (2 slots) 1724 / 1696, M=128 (4) 1950 / 1836, M=512 (16)
+// 2907 / 1945, K 2048 N 768 E 128 M=32 (2) 132 / 136 and M=64 (4) 157 / 148.
+constexpr int kDecodeMeanBf16 = 10, kDecodeMeanFp8 = 3;
+// The streaming kernels keep GEMM2's slot rows in fp32, the prefill kernels
+// of larger batches in bf16: up to this mean the rows are fp32 on both.
+constexpr int kFp32RowsMean = 16;
+
+bool mean_at_most(int64_t slots, int64_t E, int mean) {
+  const int64_t active = slots < E ? slots : E;
+  return slots <= mean * (active > 0 ? active : 1);
+}
+
 // Tile height for the fused path: 16 = decode kernels, else the prefill tile,
 // from the mean slots per expert (measured on the BASELINE shapes): bf16
-// 256-row tiles once experts average >= 256 slots, 128-row tiles from 40
-// (a half-empty 128-row tile still beats a 64-row one), else 64; 160-row
-// tiles as below.
+// 32-row tiles while they hold the mean + 2 sd of a uniform routing's
+// per-expert load (mean 22; reference sweep M=128 (mean 16) 294 us against
+// 297 with 64 rows, M=256 (32) 344 / 316); 64-row tiles up to the same bound
+// (mean 48, bf16: M=400 334 us against 338 with 128 rows, M=512 (64) 385 / 348)
+// or to mean 39 (fp8); bf16 256-row tiles once experts average >= 256 slots,
+// otherwise 128, or 160 as below.
 int choose_block_m(int wtype, int64_t M, int k, int E, int path) {
   const int64_t slots = M * k;
-  const int64_t active = slots < E ? slots : E;
   if (decode_only(wtype) || path == 2) return kDecodeBM;
-  if (path != 1 && slots <= kDecodeBM * (active > 0 ? active : 1)) return kDecodeBM;
+  if (path != 1 && mean_at_most(slots, E, wtype == FMOE_W_FP8 ? kDecodeMeanFp8 : kDecodeMeanBf16))
+    return kDecodeBM;
   const int64_t mean = slots / E;
-  if (wtype == FMOE_W_BF16 && mean >= 256) return 256;
-  if (mean < 40) return 64;
-  if (wtype == FMOE_W_FP8 || wtype == FMOE_W_BF16) {
-    // 160-row tiles where they need fewer M-tiles per expert than 128-row
-    // ones at the mean + 2 sd of a uniform routing's per-expert load (each
-    // M-tile streams the expert's whole weight panel again)
-    const double q = static_cast<double>(mean) + 2.0 * std::sqrt(static_cast<double>(mean));
-    if (std::ceil(q / 160.0) < std::ceil(q / 128.0)) return 160;
+  if (wtype == FMOE_W_BF16) {
+    if (mean >= 256) return 256;
+    if (mean <= 22) return 32;
+    if (mean <= 48) return 64;
+  } else if (mean < 40) {
+    return 64;
   }
+  // 160-row tiles where they need fewer M-tiles per expert than 128-row ones
+  // at the mean + 2 sd (each M-tile streams the expert's whole weight panel again)
+  const double q = static_cast<double>(mean) + 2.0 * std::sqrt(static_cast<double>(mean));
+  if (std::ceil(q / 160.0) < std::ceil(q / 128.0)) return 160;
   return 128;
 }
+
+// Width of a prefill output tile (the configurations of launch_prefill; the
+// fp8 160-row GEMM2's 384 columns make fewer tiles than this says).
+int prefill_bn(int wtype, int bm) { return wtype == FMOE_W_BF16 && bm <= 64 ? 128 : kPrefillBN; }
 
 // The 160-row fp8 tile stages the weight scales of at most 64 reduction
 // blocks (K, N <= 8192); larger fp8 layers take 128-row tiles.
@@ -355,7 +381,7 @@ int gemm2_impl(int wtype, const void* act, const float* act_scale, const void* w
   p.tile_lut = tile_lut;
   // fused prefill: tail split instead of split-K planes (the launcher turns
   // it off when the buffer or the runtime's occupancy query falls short)
-  p.tail_split = (tail_part && !is_decode(r) && p.y_bf16) ? kTailMaxSplit : 0;
+  p.tail_split = (tail_part && !is_decode(r) && splits == 1) ? kTailMaxSplit : 0;
   p.tail_part = tail_part;
   p.tail_bytes = tail_bytes;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -413,7 +439,10 @@ bool fused_int4_route(const fmoe_fused_args* a, int bm) {
 FusedLayout layout(const fmoe_fused_args* a) {
   FusedLayout L{};
   const int64_t slots = a->M * a->top_k;
-  L.bm = fit_block_m(a->wtype, choose_block_m(a->wtype, a->M, a->top_k, a->E, a->path), a->K, a->N);
+  // expert parallel: a local expert's share of the slots follows from the
+  // global expert count (the other ranks' experts take the rest)
+  const int experts = a->expert_map && a->n_global > a->E ? a->n_global : a->E;
+  L.bm = fit_block_m(a->wtype, choose_block_m(a->wtype, a->M, a->top_k, experts, a->path), a->K, a->N);
   L.max_tiles = fmoe_max_tiles(slots, a->E);
   fmoe_routing r{};
   r.n_tokens = a->M;
@@ -459,11 +488,12 @@ FusedLayout layout(const fmoe_fused_args* a) {
   L.actq = take(fp8 ? slots * a->N : 0);
   L.acts = take(fp8 ? 4 * slots * (a->N / 128) : 0);
   // prefill with one split: bf16 rows (see fused path); otherwise fp32 planes
-  L.y_bf16 = L.bm != kDecodeBM && L.splits == 1;
+  L.y_bf16 = L.bm != kDecodeBM && L.splits == 1 && !mean_at_most(slots, a->E, kFp32RowsMean);
   L.y = take((L.y_bf16 ? 2 : 4) * static_cast<size_t>(L.splits) * slots * a->K);
-  // prefill: logical-tile table, shared by the two GEMM launches (stream order)
-  const int64_t nn1 = (a->N + kPrefillBN / 2 - 1) / (kPrefillBN / 2);
-  const int64_t nn2 = (a->K + kPrefillBN - 1) / kPrefillBN;
+  // prefill: tile table, shared by the two GEMM launches (stream order)
+  const int bn = prefill_bn(a->wtype, L.bm);
+  const int64_t nn1 = (a->N + bn / 2 - 1) / (bn / 2);
+  const int64_t nn2 = (a->K + bn - 1) / bn;
   L.lut = take(L.bm == kDecodeBM ? 0
                                  : 16 * static_cast<size_t>(prefill_max_tiles(slots, a->E, L.bm)) * (nn1 > nn2 ? nn1 : nn2));
   L.tail = take(L.tail_bytes);
@@ -699,7 +729,8 @@ extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
   const float* acts = actqs;
   // Prefill without split-K keeps each slot's GEMM2 row in bf16 until the
   // top-k sum (SGLang's per-slot intermediate has the same rounding point);
-  // split-K planes and the decode path stay fp32.
+  // split-K planes, the decode path and batches of up to kFp32RowsMean slots
+  // per expert stay fp32.
   if (int st = gemm2_impl(a->wtype, act, acts, a->w2, a->w2_scale, a->w2_zero, a->K, a->N, &r,
                           !a->apply_router_weight_on_input, a->b2, at(L.y), L.splits, 0, lut,
                           L.y_bf16, stream, L.tail_bytes ? static_cast<float*>(at(L.tail)) : nullptr,

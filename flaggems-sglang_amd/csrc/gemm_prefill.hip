@@ -1,15 +1,15 @@
 // Prefill grouped GEMM: one expert per M-tile; MFMA tiles fed from a ring of
 // LDS stages filled by direct-to-LDS DMA.
 //
-// Workgroup = 8 waves (512 threads) laid out WAVES_M x WAVES_N; tile BM x BN;
-// SB bytes of the reduction dim per row per stage (bf16: SB = 64 or 128 ->
-// one or two v_mfma_f32_16x16x32_bf16 steps; fp8: SB = 128 -> one 128-wide
-// scale block, one v_mfma_f32_16x16x128_f8f6f4 with its result scaled by
-// a_scale[row] * w_scale[block] into the fp32 accumulator).
+// Workgroup = 4 or 8 waves laid out WAVES_M x WAVES_N; tile BM x BN; SB = 128
+// bytes of the reduction dim per row per stage (bf16: two
+// v_mfma_f32_16x16x32_bf16 steps; fp8: one 128-wide scale block, one
+// v_mfma_f32_16x16x128_f8f6f4 with its result scaled by a_scale[row] *
+// w_scale[block] into the fp32 accumulator).
 //
 // Measured on MI355X, which is what the structure follows:
 //  * DMA: global_load_lds_dwordx4 delivers ~2x the bytes per clock when
-//    consecutive lanes read one row's contiguous bytes (4 or 8 lanes x 16 B)
+//    consecutive lanes read one row's contiguous bytes (8 lanes x 16 B)
 //    than when every lane reads a different row.  LDS: a ds_read_b128
 //    fragment read runs at full rate only if each 8 consecutive lanes hit 8
 //    distinct 16-byte columns of a 128-byte window.  A stage is therefore a
@@ -51,9 +51,9 @@ constexpr int kGroupTiles = 32;   // tiles per rasterization window (~ one XCD's
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int SB_, int NBUF_, bool FP8_, Mode MODE_>
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int NBUF_, bool FP8_, Mode MODE_>
 struct Cfg {
-  static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, SB = SB_,
+  static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, SB = 128,
                        NBUF = NBUF_;
   static constexpr bool FP8 = FP8_;
   static constexpr Mode MODE = MODE_;
@@ -61,7 +61,6 @@ struct Cfg {
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   static constexpr int MI = WM / 16, NI = WN / 16;
   static constexpr int UPB = SB / 64;                       // units per 16-row block
-  static_assert(SB == 64 || SB == 128, "stage width");
   static constexpr int A_UNITS = (BM / 16) * UPB, B_UNITS = (BN / 16) * UPB;
   // unit u of a stage is DMAed by wave u % NW: waves below REM (or all of
   // them when REM == 0) issue UPW units per stage, the others UPW - 1
@@ -81,7 +80,6 @@ struct Cfg {
       NBUF * STAGE + NBUF * BM * 4 + WAVES_N * 2 * kMaxKStages * 4 <= 160 * 1024 ? kMaxKStages : 64;
   static_assert(BM % 16 == 0 && (A_UNITS % 2) == 0, "16-row blocks");
   static_assert(REM == 0 || REM <= SA_FIRST || !FP8, "a-scale waves carry the fewer units");
-  static_assert(!FP8 || SB == 128, "fp8 stages hold one 128-wide scale block");
   static_assert(MODE != Mode::kGemm1Silu || NI % 2 == 0, "gate/up pairing needs even NI");
   static_assert(NBUF >= 2 && NBUF <= 4, "ring depth");
   static_assert(NBUF * STAGE + NBUF * BM * 4 + WAVES_N * 2 * KST * 4 <= 160 * 1024, "LDS budget");
@@ -122,23 +120,17 @@ __device__ __forceinline__ void dma4(const float* g, float* l) {
                :: "v"(g), "s"(m0) : "memory", "m0");
 }
 
-// LDS unit layouts (1 KiB = one DMA wave-instruction, lane i -> bytes 16i):
-//  * 64-byte stages: a unit is 16 rows x 64 bytes; DMA lane i reads row i / 4,
-//    chunk (i % 4) ^ ((row / 2) % 4), so 4 consecutive lanes read one row's 64
-//    contiguous bytes.
-//  * 128-byte stages: a unit is 8 rows x 128 bytes (rows 0-7 or 8-15 of a
-//    16-row block); DMA lane i reads row i / 8, chunk (i % 8) ^ (row), so 8
-//    consecutive lanes read one row's 128 contiguous bytes.
-// The MFMA fragment of lane L is row L % 16, 16-byte chunk c (c = L / 16, and
-// for 128-byte stages also 4 + L / 16); with the swizzles above every 8
-// consecutive lanes of a fragment read hit 8 distinct 16-byte columns of a
-// 128-byte window, which ds_read_b128 serves at the contiguous rate
-// (measured: plain row-major or a (row / 4) swizzle run at 70% of it).
-template <int SB>
+// LDS unit layout (1 KiB = one DMA wave-instruction, lane i -> bytes 16i): a
+// unit is 8 rows x 128 bytes (rows 0-7 or 8-15 of a 16-row block); DMA lane i
+// reads row i / 8, chunk (i % 8) ^ (row), so 8 consecutive lanes read one
+// row's 128 contiguous bytes.
+// The MFMA fragment of lane L is row L % 16, 16-byte chunk c (c = L / 16 and
+// 4 + L / 16); with the swizzle every 8 consecutive lanes of a fragment read
+// hit 8 distinct 16-byte columns of a 128-byte window, which ds_read_b128
+// serves at the contiguous rate (measured: plain row-major or a (row / 4)
+// swizzle run at 70% of it).
 __device__ __forceinline__ int frag_off(int L, int c) {
-  const int r = L & 15;
-  if constexpr (SB == 64) return 16 * (4 * r + (c ^ ((r >> 1) & 3)));
-  const int ru = r & 7;
+  const int r = L & 15, ru = r & 7;
   return (r >> 3) * 1024 + 16 * (8 * ru + (c ^ ru));
 }
 
@@ -250,7 +242,7 @@ __global__ __launch_bounds__(256) void tile_lut_kernel(GemmParams p) {
 }
 
 // Adds the tail-split partials of each split tile in split order and writes
-// the tile's bf16 rows (y_bf16 layout [slot][Nout]): one workgroup per (XCD,
+// the tile's rows (bf16 or fp32, [slot][Nout]): one workgroup per (XCD,
 // tail tile, 16-row chunk), every partial of the chunk loaded before the
 // adds.  Bias and routing weight are already in the partials.
 constexpr int kFoldRows = 16;
@@ -301,15 +293,17 @@ __global__ __launch_bounds__(256) void tail_fold_kernel(GemmParams p, int stages
       a[v].w += b[v].w;
     }
   }
-  uint16_t* y = static_cast<uint16_t*>(p.out);
 #pragma unroll
   for (int v = 0; v < kVec; ++v) {
     const int idx = (threadIdx.x + v * 256) * 4;
     const int r = idx / BN, c = idx - (idx / BN) * BN;
     if (r0 + r >= re - rb || c >= cols) continue;
-    const uint32_t w0 = pack_bf16x2(a[v].x, a[v].y);
-    const uint32_t w1 = pack_bf16x2(a[v].z, a[v].w);
-    *reinterpret_cast<uint2*>(y + static_cast<int64_t>(rb + r0 + r) * p.Nout + c0 + c) = make_uint2(w0, w1);
+    const int64_t o = static_cast<int64_t>(rb + r0 + r) * p.Nout + c0 + c;
+    if (p.y_bf16)
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + o) =
+          make_uint2(pack_bf16x2(a[v].x, a[v].y), pack_bf16x2(a[v].z, a[v].w));
+    else
+      *reinterpret_cast<float4*>(static_cast<float*>(p.out) + o) = a[v];
   }
 }
 
@@ -416,15 +410,9 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   for (int i = 0; i < C::UPW; ++i) {
     const int u = min(NW * i + wid, C::UNITS - 1);
     const int b = u / UPB;
-    int lr, coff;  // row within the 16-row block, byte offset in the row slice
-    if constexpr (SB == 64) {
-      lr = lane >> 2;
-      coff = ((lane & 3) ^ ((lr >> 1) & 3)) * 16;
-    } else {
-      const int ru = lane >> 3;
-      lr = (u % 2) * 8 + ru;
-      coff = ((lane & 7) ^ ru) * 16;
-    }
+    const int ru = lane >> 3;
+    const int lr = (u % 2) * 8 + ru;               // row within the 16-row block
+    const int coff = ((lane & 7) ^ ru) * 16;       // byte offset in the row slice
     loff[i] = u * kUnit;
     if (u < C::A_UNITS) {
       src[i] = p.A + a_src_row(b * 16 + lr) * kbytes + static_cast<int64_t>(k0) * SB + coff;
@@ -474,8 +462,8 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     for (int j = 0; j < NI; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // per-lane fragment offsets within a 16-row block's units
-  const int foff0 = frag_off<SB>(lane, lane >> 4);
-  const int foff1 = SB == 64 ? 0 : frag_off<SB>(lane, 4 + (lane >> 4));
+  const int foff0 = frag_off(lane, lane >> 4);
+  const int foff1 = frag_off(lane, 4 + (lane >> 4));
   // DMA instructions per stage for this wave: its operand units, plus one
   // a-scale load
   const int per = __builtin_popcount(units) + (sa_wave ? 1 : 0);
@@ -581,12 +569,12 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     // operand line an L2 hit 1519 us, without the DMA 1353 us, without
     // fragment reads as well 1230 us, the MFMAs alone 1.0 ms at 2.07 GHz.
     constexpr int kMfma = MI * NI, NF = MI + NI;
-    constexpr int kRd = 2 * NF <= kMfma ? 2 : 1;  // MFMAs between fragment reads
-    // ... and between DMA units (2 / 3 / 4 measured at 256 x 256: Mixtral
-    // M=4096 2607 / 2562 / 2610 us a call; issued back to back they hold up
-    // the MFMAs, further apart they arrive late for a 2-deep ring)
-    constexpr int kDma = 3 * C::UPW <= kMfma ? 3 : (2 * C::UPW <= kMfma ? 2 : 1);
-    static_assert(NF <= kMfma && C::UPW <= kMfma, "reads and DMA fit between the MFMAs of a step");
+    // The f-th of n reads (DMA units) goes before MFMA at(f, n, gap): every
+    // second MFMA for reads, every third for DMA units (2 / 3 / 4 measured at
+    // 256 x 256: Mixtral M=4096 2607 / 2562 / 2610 us a call; back to back
+    // they hold up the MFMAs, further apart they arrive late for a 2-deep
+    // ring), closer where a step has too few MFMAs for that.
+    auto at = [](int f, int n, int gap) { return gap * n <= kMfma ? gap * f : f * kMfma / n; };
     bf16x8_t fa[2][MI], fb[2][NI];
     // fragment f of step h of the stage in slot st, into register set q
     auto read_frag = [&](const uint8_t* st, int h, int q, int f) {
@@ -605,10 +593,16 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
       for (int m = 0; m < kMfma; ++m) {
         const int i = m / NI, j = m % NI;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (READ)
-          if (m % kRd == 0 && m / kRd < NF) read_frag(st, h, 1 - q, m / kRd);
-        if constexpr (DMA)
-          if (m % kDma == 0 && m / kDma < C::UPW) issue_unit(kd, m / kDma);
+        if constexpr (READ) {
+#pragma unroll
+          for (int f = 0; f < NF; ++f)
+            if (at(f, NF, 2) == m) read_frag(st, h, 1 - q, f);
+        }
+        if constexpr (DMA) {
+#pragma unroll
+          for (int u = 0; u < C::UPW; ++u)
+            if (at(u, C::UPW, 3 * C::UPW <= kMfma ? 3 : 2) == m) issue_unit(kd, u);
+        }
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[q][j], fa[q][i], acc[i][j], 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -631,43 +625,21 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
     } else if (nk > 0) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) read_frag(lds[0], 0, 0, f);
-      if constexpr (UPB == 2) {
-        int kt = 0;
-        for (; kt + NBUF < nk; ++kt) {
-          step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
-          done_reading();
-          wait_full(Ring2{});
-          step(1, T{}, lds[(kt + 1) % NBUF], 0, T{}, kt + NBUF);
-        }
-        for (; kt + 1 < nk; ++kt) {
-          step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
-          done_reading();
-          wait_stage(min(NBUF - 2, nk - 2 - kt));
-          step(1, T{}, lds[(kt + 1) % NBUF], 0, F{}, 0);
-        }
+      int kt = 0;
+      for (; kt + NBUF < nk; ++kt) {
         step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
-        step(1, F{}, nullptr, 0, F{}, 0);
-      } else {
-        // one step per stage: the register sets alternate with the stages
-        auto stage = [&](int kt, int q) {
-          if (kt + 1 < nk) {
-            done_reading();
-            if (kt + NBUF < nk) {
-              wait_full(Ring2{});
-              step(q, T{}, lds[(kt + 1) % NBUF], 0, T{}, kt + NBUF);
-            } else {
-              wait_stage(min(NBUF - 2, nk - 2 - kt));
-              step(q, T{}, lds[(kt + 1) % NBUF], 0, F{}, 0);
-            }
-          } else {
-            step(q, F{}, nullptr, 0, F{}, 0);
-          }
-        };
-        for (int kt = 0; kt < nk; kt += 2) {
-          stage(kt, 0);
-          if (kt + 1 < nk) stage(kt + 1, 1);
-        }
+        done_reading();
+        wait_full(Ring2{});
+        step(1, T{}, lds[(kt + 1) % NBUF], 0, T{}, kt + NBUF);
       }
+      for (; kt + 1 < nk; ++kt) {
+        step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
+        done_reading();
+        wait_stage(min(NBUF - 2, nk - 2 - kt));
+        step(1, T{}, lds[(kt + 1) % NBUF], 0, F{}, 0);
+      }
+      step(0, T{}, lds[kt % NBUF], 1, F{}, 0);
+      step(1, F{}, nullptr, 0, F{}, 0);
     }
   }
 
@@ -889,7 +861,7 @@ int launch(const GemmParams& p0, hipStream_t s) {
     const int slots = xcd_slots<C>();
     const int64_t pairs = tail_pairs_for<C>(p.max_tiles, p.Nout);
     p.tail_pairs = static_cast<int64_t>(p.tail_bytes / (static_cast<size_t>(C::BM) * C::BN * sizeof(float)));
-    if (slots <= 0 || !p.tail_part || pairs <= 0 || p.tail_pairs < pairs || p.splits != 1 || !p.y_bf16) {
+    if (slots <= 0 || !p.tail_part || pairs <= 0 || p.tail_pairs < pairs || p.splits != 1) {
       p.tail_split = 0;  // whole tiles only
     } else {
       p.tail_slots = slots;
@@ -927,7 +899,13 @@ int launch(const GemmParams& p0, hipStream_t s) {
 //   bf16: BM 256 -> 256x256, 4x2 waves, 128-byte stages, 2-deep ring
 //         BM 160 -> 160x256, 2x4 waves, 128-byte stages, 3-deep ring
 //         BM 128 -> 128x256, 2x4 waves, 128-byte stages, 3-deep ring
-//         BM  64 ->  64x256, 1x4 waves, 64-byte stages, 4-deep ring
+//         BM  64 ->  64x128, 1x4 waves, 128-byte stages, 3-deep ring
+//         BM  32 ->  32x128, 1x4 waves, 128-byte stages, 4-deep ring
+//         (72 and 80 KiB of LDS: two workgroups per CU, so one streams while
+//         the other starts or ends, with 48 / 60 KiB each in flight; 64x256
+//         with 64-byte stages in a 4-deep ring, one workgroup per CU, took 346
+//         us against 297 on the reference sweep's M=128, 563 against 501 on
+//         Mixtral M=100)
 //   fp8 : BM 160 -> GEMM1 160x256, 3-deep ring; GEMM2 160x384, 2-deep ring;
 //                   2x4 waves, 128-byte stages (K, N <= 8192)
 //         BM 128 -> 128x256, 2x4 waves, 128-byte stages, 3-deep ring
@@ -935,22 +913,24 @@ int launch(const GemmParams& p0, hipStream_t s) {
 int launch_prefill(WType wt, Mode mode, int bm, const GemmParams& p, hipStream_t s) {
   using namespace prefill;
   const bool fp8 = wt == WType::kFp8;
-#define L(BM, BN, WMS, WNS, SB, NB, F8)                                                      \
-  (mode == Mode::kGemm1Silu ? launch<Cfg<BM, BN, WMS, WNS, SB, NB, F8, Mode::kGemm1Silu>>(p, s) \
-                            : launch<Cfg<BM, BN, WMS, WNS, SB, NB, F8, Mode::kGemm2>>(p, s))
+#define L(BM, BN, WMS, WNS, NB, F8)                                                          \
+  (mode == Mode::kGemm1Silu ? launch<Cfg<BM, BN, WMS, WNS, NB, F8, Mode::kGemm1Silu>>(p, s) \
+                            : launch<Cfg<BM, BN, WMS, WNS, NB, F8, Mode::kGemm2>>(p, s))
   if (!fp8) {
-    if (bm == 256) return L(256, 256, 4, 2, 128, 2, false);
-    if (bm == 160) return L(160, 256, 2, 4, 128, 3, false);
-    if (bm == 128) return L(128, 256, 2, 4, 128, 3, false);
-    if (bm == 64) return L(64, 256, 1, 4, 64, 4, false);
+    if (bm == 256) return L(256, 256, 4, 2, 2, false);
+    if (bm == 160) return L(160, 256, 2, 4, 3, false);
+    if (bm == 128) return L(128, 256, 2, 4, 3, false);
+    if (bm == 64) return L(64, 128, 1, 4, 3, false);
+    if (bm == 32) return L(32, 128, 1, 4, 4, false);
   } else {
     // GEMM2 with 160-row tiles: 384-wide output tiles (2-deep ring of 68 KiB
     // stages), so the activation tile is re-read by a third fewer N-tiles
     // (13% fewer operand requests per output; DSV3 GEMM2 M=4096 -5%, M=8192 -7%)
-    if (bm == 160 && mode == Mode::kGemm2) return launch<Cfg<160, 384, 2, 4, 128, 2, true, Mode::kGemm2>>(p, s);
-    if (bm == 160) return L(160, 256, 2, 4, 128, 3, true);
-    if (bm == 128) return L(128, 256, 2, 4, 128, 3, true);
-    if (bm == 64) return L(64, 256, 1, 8, 128, 3, true);
+    if (bm == 160)
+      return mode == Mode::kGemm2 ? launch<Cfg<160, 384, 2, 4, 2, true, Mode::kGemm2>>(p, s)
+                                  : launch<Cfg<160, 256, 2, 4, 3, true, Mode::kGemm1Silu>>(p, s);
+    if (bm == 128) return L(128, 256, 2, 4, 3, true);
+    if (bm == 64) return L(64, 256, 1, 8, 3, true);
   }
 #undef L
   return fmoe_host::fail(FMOE_ERR_UNSUPPORTED,
@@ -961,18 +941,19 @@ int launch_prefill(WType wt, Mode mode, int bm, const GemmParams& p, hipStream_t
 // weight type and tile height (the configuration launch_prefill picks).
 size_t prefill_tail_bytes(WType wt, int bm, int64_t max_tiles, int64_t Nout) {
   using namespace prefill;
-#define T(BM, BN, WMS, WNS, SB, NB, F8) \
-  static_cast<size_t>(tail_pairs_for<Cfg<BM, BN, WMS, WNS, SB, NB, F8, Mode::kGemm2>>(max_tiles, Nout)) * BM * BN * 4
+#define T(BM, BN, WMS, WNS, NB, F8) \
+  static_cast<size_t>(tail_pairs_for<Cfg<BM, BN, WMS, WNS, NB, F8, Mode::kGemm2>>(max_tiles, Nout)) * BM * BN * 4
   if (wt != WType::kFp8) {
     if (wt != WType::kBf16) return 0;
-    if (bm == 256) return T(256, 256, 4, 2, 128, 2, false);
-    if (bm == 160) return T(160, 256, 2, 4, 128, 3, false);
-    if (bm == 128) return T(128, 256, 2, 4, 128, 3, false);
-    if (bm == 64) return T(64, 256, 1, 4, 64, 4, false);
+    if (bm == 256) return T(256, 256, 4, 2, 2, false);
+    if (bm == 160) return T(160, 256, 2, 4, 3, false);
+    if (bm == 128) return T(128, 256, 2, 4, 3, false);
+    if (bm == 64) return T(64, 128, 1, 4, 3, false);
+    if (bm == 32) return T(32, 128, 1, 4, 4, false);
   } else {
-    if (bm == 160) return T(160, 384, 2, 4, 128, 2, true);
-    if (bm == 128) return T(128, 256, 2, 4, 128, 3, true);
-    if (bm == 64) return T(64, 256, 1, 8, 128, 3, true);
+    if (bm == 160) return T(160, 384, 2, 4, 2, true);
+    if (bm == 128) return T(128, 256, 2, 4, 3, true);
+    if (bm == 64) return T(64, 256, 1, 8, 3, true);
   }
 #undef T
   return 0;

@@ -247,8 +247,8 @@ int fmoe_gemm2_ex(int wtype, const void* act, const float* act_scale, const void
                   int path, void* stream);
 
 /* Tile height the library pairs with the GEMM kernels for a problem size:
- * 16 selects the decode (streaming) kernels, 64 / 128 / 160 / 256 the prefill
- * kernels (256: bf16 only; 160 with fp8 weights needs K and N <= 8192 -- the
+ * 16 selects the decode (streaming) kernels, 32 / 64 / 128 / 160 / 256 the prefill
+ * kernels (32 and 256: bf16 only; 160 with fp8 weights needs K and N <= 8192 -- the
  * caller substitutes 128 above that; fmoe_fused_experts does so itself).
  * path: 0 = choose, 1 = prefill, 2 = decode (4-bit weights always report 16:
  * their large-batch route dequantizes to bf16 inside fmoe_fused_experts). */
@@ -257,7 +257,8 @@ int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path);
 /* The tile height fmoe_fused_experts uses for a layer of hidden size K and
  * intermediate size N: fmoe_choose_block_m with the fp8 160 -> 128 substitution
  * above applied (callers that build their own routing for the stage API use
- * this, so they always agree with the fused path).  Reference counterpart: the
+ * this, so they always agree with the fused path; with an expert map E is the
+ * global expert count).  Reference counterpart: the
  * block size triton_kernels' matmul_ogs picks for its routing, ops/fused_moe.py:190. */
 int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N);
 

@@ -14,7 +14,8 @@ DEV = "cuda"
 E, k = 8, 2
 
 COUNTS = {  # tile height -> slots per expert, each 1 modulo the height
-    64: [65, 65] + [1] * 6,
+    32: [33, 33] + [1] * 6,
+    64: [65, 65, 65] + [1] * 5,
     128: [129, 129, 129] + [1] * 5,
     160: [161] * 6 + [1, 1],
     256: [257] * 8,
@@ -35,8 +36,8 @@ def test_every_expert_ends_in_a_one_row_tile(bm, fp8, K, N):
     from flaggems_sglang import _lib
     from flaggems_sglang import quant as Q
 
-    if fp8 and bm == 256:
-        pytest.skip("no 256-row fp8 tiles")
+    if fp8 and bm in (32, 256):
+        pytest.skip(f"no {bm}-row fp8 tiles")
     counts = COUNTS[bm]
     ids = _ids(counts)
     M = ids.shape[0]
