@@ -7,6 +7,9 @@
 namespace fmoe {
 int launch_prefill(WType wt, Mode mode, int bm, const GemmParams& p, hipStream_t s);
 size_t prefill_tail_bytes(WType wt, int bm, int64_t max_tiles, int64_t Nout);
+int launch_w4(Mode mode, const GemmParams& p, hipStream_t s);
+size_t w4_tail_bytes(int64_t max_tiles, int64_t Nout);
+int rows_for_int4(const void* x, int64_t M, int64_t K, void* xp, float* xs, hipStream_t s);
 int decode_int4_row_split(int64_t max_tiles);
 int launch_decode(WType wt, Mode mode, const GemmParams& p, hipStream_t s);
 int launch_gemm1_token(const GemmParams& p, int E, int k, hipStream_t s);
@@ -398,6 +401,7 @@ struct FusedLayout {
   int splits;
   bool y_bf16;
   bool fused4;  // one-launch int4 decode (splits = N / 128 planes)
+  bool w4;      // int4 prefill kernels (gemm_w4.hip)
   int64_t max_tiles;
   size_t align_ws, expt_indx, expt_scal, topk_indx, gate_indx, gate_scal, hist, offs_raw,
       offs_pad, tile_map, n_tiles, xq, xs, act, actq, acts, y, lut, tail, total;
@@ -436,6 +440,45 @@ bool fused_int4_route(const fmoe_fused_args* a, int bm) {
          fused_int4_fits(a->M * a->top_k, a->K);
 }
 
+// Large batches of 4-bit weights: the decode kernels re-read an expert's
+// weights for every 16-slot tile, so once experts average kDequantMinSlots
+// slots the weights are dequantized once to bf16 (in the workspace) and the
+// bf16 prefill kernels run on them.  Measured on the Mixtral shape (tiled
+// int4, decode kernels vs dequantize + bf16 prefill): M=512 (128 slots per
+// expert) 1.16 vs 1.66 ms, M=1024 (256) 2.20 vs 2.13 ms, M=4096 8.4 vs 3.8 ms;
+// MXFP4 M=1024 2.81 vs 2.14 ms.
+constexpr int64_t kDequantMinSlots = 256;
+
+// The bf16 copies live in the caller's workspace for the duration of the
+// call (2 * E * 3 * N * K bytes: 2.8 GB for the Mixtral shape), so the route is
+// taken automatically only while they stay within kDequantMaxBytes; above it
+// (e.g. a DeepSeek-size int4 layer, ~22 GB) the decode kernels run at every M.
+// path = 1 asks for the route regardless of the size.
+constexpr size_t kDequantMaxBytes = size_t(4) << 30;
+
+// bytes of the bf16 copies of w13 and w2
+size_t dequant_bytes(const fmoe_fused_args* a) {
+  return al(2 * static_cast<size_t>(a->E) * 2 * a->N * a->K) + al(2 * static_cast<size_t>(a->E) * a->K * a->N);
+}
+
+bool dequant_prefill(const fmoe_fused_args* a) {
+  if (!decode_only(a->wtype) || a->path == 2) return false;
+  if (a->path == 1) return true;
+  return a->M * a->top_k >= kDequantMinSlots * a->E && dequant_bytes(a) <= kDequantMaxBytes;
+}
+
+// int4 batches between the two run on the prefill kernels that unpack the
+// nibbles in registers (gemm_w4.hip; path 1 keeps asking for the bf16 copies).
+// Mixtral shape, streaming kernels / these in us a call: M=256 (64 slots per
+// expert) 421 / 421, M=500 720 / 600, M=800 1152 / 754; TP-8 M=256 104 / 121,
+// M=600 (150) 154 / 132.
+constexpr int kW4Mean = 80, kW4BM = 128;
+bool w4_route(const fmoe_fused_args* a) {
+  if (!is_int4(a->wtype) || a->activation == FMOE_ACT_SWIGLU || a->b13 || a->path != 0) return false;
+  const int experts = a->expert_map && a->n_global > a->E ? a->n_global : a->E;
+  return !mean_at_most(a->M * a->top_k, experts, kW4Mean) && !dequant_prefill(a);
+}
+
 FusedLayout layout(const fmoe_fused_args* a) {
   FusedLayout L{};
   const int64_t slots = a->M * a->top_k;
@@ -443,6 +486,8 @@ FusedLayout layout(const fmoe_fused_args* a) {
   // global expert count (the other ranks' experts take the rest)
   const int experts = a->expert_map && a->n_global > a->E ? a->n_global : a->E;
   L.bm = fit_block_m(a->wtype, choose_block_m(a->wtype, a->M, a->top_k, experts, a->path), a->K, a->N);
+  L.w4 = w4_route(a);
+  if (L.w4) L.bm = kW4BM;
   L.max_tiles = fmoe_max_tiles(slots, a->E);
   fmoe_routing r{};
   r.n_tokens = a->M;
@@ -463,6 +508,11 @@ FusedLayout layout(const fmoe_fused_args* a) {
                   (a->wtype == FMOE_W_BF16 || a->wtype == FMOE_W_FP8))
                      ? prefill_tail_bytes(to_wt(a->wtype), L.bm, prefill_max_tiles(slots, a->E, L.bm), a->K)
                      : 0;
+  // int4: few output tiles, each part of a split at least 8 groups
+  const int64_t w4_wgs = (slots + L.bm - 1) / L.bm * ((a->K + kPrefillBN - 1) / kPrefillBN);
+  if (L.w4) L.splits = 1;
+  if (L.w4 && w4_wgs < kPrefillNoSplitWgs && a->N / 128 >= 8 * kTailMaxSplit)
+    L.tail_bytes = w4_tail_bytes(prefill_max_tiles(slots, a->E, L.bm), a->K);
   if (L.tail_bytes > 0) L.splits = 1;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -482,13 +532,15 @@ FusedLayout layout(const fmoe_fused_args* a) {
   L.tile_map = take(4 * L.max_tiles);
   L.n_tiles = take(4);
   const bool fp8 = a->wtype == FMOE_W_FP8 && L.bm != kDecodeBM;
-  L.xq = take(fp8 ? a->M * a->K : 0);
-  L.xs = take(fp8 ? 4 * a->M * (a->K / 128) : 0);
+  // fp8: codes and scales of x; int4 prefill: x in the nibble order, group sums
+  L.xq = take(fp8 ? a->M * a->K : (L.w4 ? 2 * a->M * a->K : 0));
+  L.xs = take(fp8 || L.w4 ? 4 * a->M * (a->K / 128) : 0);
   L.act = take(fp8 ? 0 : 2 * slots * a->N);  // fp8 prefill: GEMM1 writes the quantized act
   L.actq = take(fp8 ? slots * a->N : 0);
-  L.acts = take(fp8 ? 4 * slots * (a->N / 128) : 0);
+  L.acts = take(fp8 || L.w4 ? 4 * slots * (a->N / 128) : 0);
   // prefill with one split: bf16 rows (see fused path); otherwise fp32 planes
-  L.y_bf16 = L.bm != kDecodeBM && L.splits == 1 && !mean_at_most(slots, a->E, kFp32RowsMean);
+  // (the int4 prefill kernels' rows are fp32, as the streaming kernels' are)
+  L.y_bf16 = L.bm != kDecodeBM && !L.w4 && L.splits == 1 && !mean_at_most(slots, a->E, kFp32RowsMean);
   L.y = take((L.y_bf16 ? 2 : 4) * static_cast<size_t>(L.splits) * slots * a->K);
   // prefill: tile table, shared by the two GEMM launches (stream order)
   const int bn = prefill_bn(a->wtype, L.bm);
@@ -585,33 +637,6 @@ int fused_tiny(const fmoe_fused_args* a, const FusedLayout& L, char* ws, hipStre
 
 }  // namespace
 
-// Large batches of 4-bit weights: the decode kernels re-read an expert's
-// weights for every 16-slot tile, so once experts average kDequantMinSlots
-// slots the weights are dequantized once to bf16 (in the workspace) and the
-// bf16 prefill kernels run on them.  Measured on the Mixtral shape (tiled
-// int4, decode kernels vs dequantize + bf16 prefill): M=512 (128 slots per
-// expert) 1.16 vs 1.66 ms, M=1024 (256) 2.20 vs 2.13 ms, M=4096 8.4 vs 3.8 ms;
-// MXFP4 M=1024 2.81 vs 2.14 ms.
-constexpr int64_t kDequantMinSlots = 256;
-
-// The bf16 copies live in the caller's workspace for the duration of the
-// call (2 * E * 3 * N * K bytes: 2.8 GB for the Mixtral shape), so the route is
-// taken automatically only while they stay within kDequantMaxBytes; above it
-// (e.g. a DeepSeek-size int4 layer, ~22 GB) the decode kernels run at every M.
-// path = 1 asks for the route regardless of the size.
-constexpr size_t kDequantMaxBytes = size_t(4) << 30;
-
-// bytes of the bf16 copies of w13 and w2
-size_t dequant_bytes(const fmoe_fused_args* a) {
-  return al(2 * static_cast<size_t>(a->E) * 2 * a->N * a->K) + al(2 * static_cast<size_t>(a->E) * a->K * a->N);
-}
-
-bool dequant_prefill(const fmoe_fused_args* a) {
-  if (!decode_only(a->wtype) || a->path == 2) return false;
-  if (a->path == 1) return true;
-  return a->M * a->top_k >= kDequantMinSlots * a->E && dequant_bytes(a) <= kDequantMaxBytes;
-}
-
 // The same call on bf16 copies of the weights placed at the workspace start.
 fmoe_fused_args bf16_args(const fmoe_fused_args* a, void* ws) {
   fmoe_fused_args b = *a;
@@ -707,6 +732,25 @@ extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
     x = at(L.xq);
     xs = static_cast<const float*>(at(L.xs));
   }
+  if (L.w4) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    float* xsum = static_cast<float*>(at(L.xs));
+    if (int st = rows_for_int4(a->x, a->M, a->K, at(L.xq), xsum, s)) return st;
+    GemmParams g1 = base_params(&r), g2;
+    decode_pair(a, L, ws, g1, g2);
+    g1.A = static_cast<const uint8_t*>(at(L.xq));
+    g1.a_scale = xsum;
+    g1.act_qs = static_cast<float*>(at(L.acts));
+    g2.a_scale = g1.act_qs;
+    g1.tile_lut = g2.tile_lut = static_cast<int4*>(at(L.lut));
+    g2.tail_split = L.tail_bytes ? kTailMaxSplit : 0;
+    g2.tail_part = static_cast<float*>(at(L.tail));
+    g2.tail_bytes = L.tail_bytes;
+    if (int st = launch_w4(Mode::kGemm1Silu, g1, s)) return st;
+    if (int st = launch_w4(Mode::kGemm2, g2, s)) return st;
+    return fmoe_moe_sum(static_cast<const float*>(at(L.y)), 1, o.gate_indx, a->M, a->top_k, a->K,
+                        a->routed_scaling_factor, a->out, stream);
+  }
   if (L.fused4) {
     GemmParams g1 = base_params(&r), g2;
     decode_pair(a, L, ws, g1, g2);
@@ -780,7 +824,14 @@ int scratch_for_current_device(void** out) {
 
 extern "C" int fmoe_fused_experts_noalloc(const fmoe_fused_args* a, void* stream) {
   if (int st = check_fused(a)) return st;
-  const size_t need = fmoe_fused_experts_workspace_bytes(a);
+  size_t need = fmoe_fused_experts_workspace_bytes(a);
+  fmoe_fused_args b = *a;
+  // batches that the streaming kernels would also take: those need less
+  if (need > FMOE_NOALLOC_SCRATCH_BYTES && a->path == 0 &&
+      (w4_route(a) || mean_at_most(a->M * a->top_k, a->E, kFp32RowsMean))) {
+    b.path = 2;
+    need = fmoe_fused_experts_workspace_bytes(&b);
+  }
   if (need > FMOE_NOALLOC_SCRATCH_BYTES)
     return fail(FMOE_ERR_UNSUPPORTED,
                 "fused_experts_noalloc: this call needs %zu bytes of workspace, above the %zu-byte "
@@ -788,7 +839,6 @@ extern "C" int fmoe_fused_experts_noalloc(const fmoe_fused_args* a, void* stream
                 need, static_cast<size_t>(FMOE_NOALLOC_SCRATCH_BYTES));
   void* ws = nullptr;
   if (int st = scratch_for_current_device(&ws)) return st;
-  fmoe_fused_args b = *a;
   b.workspace = ws;
   b.workspace_bytes = FMOE_NOALLOC_SCRATCH_BYTES;
   return fmoe_fused_experts(&b, stream);

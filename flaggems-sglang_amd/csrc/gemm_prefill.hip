@@ -40,16 +40,10 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm.hpp"
+#include "prefill.hpp"
 
 namespace fmoe {
 namespace prefill {
-
-constexpr int kUnit = 1024;       // one DMA wave-instruction: 64 lanes x 16 B
-constexpr int kMaxKStages = 128;  // fp8: reduction dims up to 16384 (64 stages when LDS is short)
-constexpr int kGroupTiles = 32;   // tiles per rasterization window (~ one XCD's CUs)
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int NBUF_, bool FP8_, Mode MODE_>
 struct Cfg {
@@ -86,227 +80,6 @@ struct Cfg {
   static_assert(SA_WAVES <= NW, "a-scale waves");
 };
 
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4) | (0xf << 8));
-}
-
-// wait until at most n of this wave's loads are in flight (n uniform, 0..MAX)
-template <int MAX>
-__device__ __forceinline__ void wait_loads(int n) {
-  if constexpr (MAX == 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (n >= MAX) wait_vmcnt<MAX>();
-    else wait_loads<MAX - 1>(n);
-  }
-}
-
-__device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" ::: "memory"); }
-
-__device__ __forceinline__ uint32_t lds_addr(const void* l) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(l)));
-}
-// lane i's 16 (or 4) bytes land at LDS address l + 16 i (4 i)
-__device__ __forceinline__ void dma16(const uint8_t* g, uint8_t* l) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_addr(l));
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :: "v"(g), "s"(m0) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const float* g, float* l) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_addr(l));
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-               :: "v"(g), "s"(m0) : "memory", "m0");
-}
-
-// LDS unit layout (1 KiB = one DMA wave-instruction, lane i -> bytes 16i): a
-// unit is 8 rows x 128 bytes (rows 0-7 or 8-15 of a 16-row block); DMA lane i
-// reads row i / 8, chunk (i % 8) ^ (row), so 8 consecutive lanes read one
-// row's 128 contiguous bytes.
-// The MFMA fragment of lane L is row L % 16, 16-byte chunk c (c = L / 16 and
-// 4 + L / 16); with the swizzle every 8 consecutive lanes of a fragment read
-// hit 8 distinct 16-byte columns of a 128-byte window, which ds_read_b128
-// serves at the contiguous rate (measured: plain row-major or a (row / 4)
-// swizzle run at 70% of it).
-__device__ __forceinline__ int frag_off(int L, int c) {
-  const int r = L & 15, ru = r & 7;
-  return (r >> 3) * 1024 + 16 * (8 * ru + (c ^ ru));
-}
-
-__device__ __forceinline__ i32x4_t lds16(const uint8_t* p) { return *reinterpret_cast<const i32x4_t*>(p); }
-
-// Expert e with offs_pad[e] * nn <= key < offs_pad[e + 1] * nn (offs_pad is
-// non-decreasing, offs_pad[0] = 0, key < offs_pad[E] * nn): two rounds of 64
-// parallel probes and a ballot, instead of a serial binary search.
-__device__ __forceinline__ int find_expert(const int32_t* offs_pad, int E, int key, int nn, int lane) {
-  const int S = (E + 1 + kWave - 1) / kWave;
-  const int i1 = min(lane * S, E);
-  uint64_t b = __ballot(offs_pad[i1] * nn <= key);
-  const int base = (63 - __builtin_clzll(b)) * S;
-  const int i2 = min(base + lane, E);
-  b = __ballot(lane < S && offs_pad[i2] * nn <= key);
-  return base + (63 - __builtin_clzll(b));
-}
-
-// Which weight row of a tile sits in row lr of its 16-row LDS block b.  The
-// MFMA takes the weight fragment as its first operand, so a lane ends with
-// four consecutive weight rows 4 * (lane / 16) + 0..3 (output columns) of one
-// slot row, lane % 16: what a row store wants, with no exchange between lanes.
-// With PAIR, the rows of blocks 2p and 2p + 1 are dealt out four by four, so
-// a lane's two blocks are 8 consecutive columns (one 16-byte bf16 store, and
-// 64 contiguous bytes per row and instruction).  fp8: one activation scale
-// per lane and row block instead of four.  Against the opposite operand order
-// with 4x4 lane transposes and integer bf16 rounding in the epilogue, outputs
-// bit-identical: Mixtral bf16 M=4096 2707 -> 2626 us a call, Qwen3 M=8192
-// 891 -> 817 us, reference sweep M=1024 436 -> 416 us, DSV3 fp8 M=4096
-// 2991 -> 2724 us.
-template <bool PAIR>
-__device__ __forceinline__ int tile_row(int b, int lr) {
-  if constexpr (PAIR) return (b >> 1) * 32 + (lr >> 2) * 8 + (b & 1) * 4 + (lr & 3);
-  return b * 16 + lr;
-}
-// First of the lane's four output columns of block j (same numbering).
-template <bool PAIR>
-__device__ __forceinline__ int tile_col(int j, int lane) {
-  return tile_row<PAIR>(j, (lane >> 4) * 4);
-}
-
-// Logical tile L (within one split) -> expert, N-tile and rows.  Per expert,
-// windows of all its T M-tiles x G N-tiles (T * G ~ group_tiles, about what
-// one XCD runs at once) are enumerated M-fastest, so the tiles that share a
-// weight panel run together on one XCD and the panel is fetched from HBM
-// once.  Called by one whole wave (find_expert ballots).
-struct Tile {
-  int e, nt, row_beg, row_end;
-};
-template <int BM>
-__device__ __forceinline__ Tile tile_of(const GemmParams& p, int L, int lane) {
-  const int nn = p.n_ntiles;
-  Tile t;
-  t.e = find_expert(p.offs_pad, p.n_experts, L, nn, lane);
-  const int t0 = p.offs_pad[t.e];
-  const int T = p.offs_pad[t.e + 1] - t0;
-  const int local = L - t0 * nn;
-  const int G = max(1, p.group_tiles / T);
-  const int grp = local / (T * G);
-  const int rr = local - grp * T * G;
-  const int blk = rr % T;
-  t.nt = grp * G + rr / T;
-  t.row_beg = p.offs_raw[t.e] + blk * BM;
-  t.row_end = min(p.offs_raw[t.e + 1], t.row_beg + BM);
-  return t;
-}
-
-// Tail split of XCD x (GEMM2, p.tail_split > 1): the XCD's logical tiles are
-// [base, base + Tx) (xcd_remap's partition of the T live tiles).  Whole
-// tiles fill rounds of `slots` workgroups; the tl = Tx % slots tiles of the
-// last partial round are split S = min(max_split, slots / tl, stages) ways,
-// so their tl * S workgroups fill at most one round.  S = 1: no split, every
-// tile whole.  The GEMM and tail_fold_kernel derive the same plan.
-struct TailPlan {
-  int base, full, tl, S;
-};
-__device__ __forceinline__ TailPlan tail_plan(int T, int x, int max_split, int slots, int stages) {
-  const int q = T / kNumXcd, r8 = T % kNumXcd;
-  const int Tx = q + (x < r8 ? 1 : 0);
-  TailPlan t;
-  t.base = x * q + min(x, r8);
-  t.tl = Tx % slots;
-  t.S = t.tl > 0 ? min(min(max_split, slots / t.tl), stages) : 1;
-  if (t.S < 2) {
-    t.S = 1;
-    t.tl = 0;
-  }
-  t.full = Tx - t.tl;
-  return t;
-}
-// Index of XCD x's first tail pair: the pairs of XCDs 0 .. x-1 come first.
-__device__ __forceinline__ int tail_offset(int T, int x, int max_split, int slots, int stages) {
-  int off = 0;
-  for (int y = 0; y < x; ++y) {
-    const TailPlan t = tail_plan(T, y, max_split, slots, stages);
-    off += t.tl * t.S;
-  }
-  return off;
-}
-
-// Fills p.tile_lut for every live logical tile: one wave per tile.
-template <int BM>
-__global__ __launch_bounds__(256) void tile_lut_kernel(GemmParams p) {
-  const int lane = threadIdx.x % kWave;
-  const int L = blockIdx.x * 4 + threadIdx.x / kWave;
-  if (L >= *p.n_tiles * p.n_ntiles) return;
-  const Tile t = tile_of<BM>(p, L, lane);
-  if (lane == 0) p.tile_lut[L] = int4{t.e, t.nt, t.row_beg, t.row_end};
-}
-
-// Adds the tail-split partials of each split tile in split order and writes
-// the tile's rows (bf16 or fp32, [slot][Nout]): one workgroup per (XCD,
-// tail tile, 16-row chunk), every partial of the chunk loaded before the
-// adds.  Bias and routing weight are already in the partials.
-constexpr int kFoldRows = 16;
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void tail_fold_kernel(GemmParams p, int stages) {
-  constexpr int kChunks = BM / kFoldRows;
-  constexpr int kVec = kFoldRows * BN / (4 * 256);  // float4 per thread and partial
-  static_assert(kFoldRows * BN % (4 * 256) == 0, "fold chunk");
-  const int rc = blockIdx.x % kChunks;
-  const int xt = blockIdx.x / kChunks;
-  const int x = xt / p.tail_slots, t = xt % p.tail_slots;
-  const int T = *p.n_tiles * p.n_ntiles;
-  const TailPlan pl = tail_plan(T, x, p.tail_split, p.tail_slots, stages);
-  if (t >= pl.tl) return;
-  const int pair0 = tail_offset(T, x, p.tail_split, p.tail_slots, stages) + t * pl.S;
-  if (pair0 + pl.S > p.tail_pairs) return;
-  const int L = pl.base + pl.full + t;
-  int nt, rb, re;
-  if (p.tile_lut) {
-    const int4 v = p.tile_lut[L];
-    nt = v.y;
-    rb = v.z;
-    re = v.w;
-  } else {
-    const Tile tt = tile_of<BM>(p, L, threadIdx.x % kWave);
-    nt = tt.nt;
-    rb = tt.row_beg;
-    re = tt.row_end;
-  }
-  const int r0 = rc * kFoldRows;
-  if (r0 >= re - rb) return;
-  const int64_t c0 = static_cast<int64_t>(nt) * BN;
-  const int cols = static_cast<int>(min(static_cast<int64_t>(BN), p.Nout - c0));
-  const float* part = p.tail_part + static_cast<int64_t>(pair0) * (BM * BN) + r0 * BN;
-  float4 a[kVec];
-#pragma unroll
-  for (int v = 0; v < kVec; ++v) a[v] = *reinterpret_cast<const float4*>(part + (threadIdx.x + v * 256) * 4);
-  for (int sp = 1; sp < pl.S; ++sp) {
-    float4 b[kVec];
-#pragma unroll
-    for (int v = 0; v < kVec; ++v)
-      b[v] = *reinterpret_cast<const float4*>(part + static_cast<int64_t>(sp) * (BM * BN) + (threadIdx.x + v * 256) * 4);
-#pragma unroll
-    for (int v = 0; v < kVec; ++v) {
-      a[v].x += b[v].x;
-      a[v].y += b[v].y;
-      a[v].z += b[v].z;
-      a[v].w += b[v].w;
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < kVec; ++v) {
-    const int idx = (threadIdx.x + v * 256) * 4;
-    const int r = idx / BN, c = idx - (idx / BN) * BN;
-    if (r0 + r >= re - rb || c >= cols) continue;
-    const int64_t o = static_cast<int64_t>(rb + r0 + r) * p.Nout + c0 + c;
-    if (p.y_bf16)
-      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + o) =
-          make_uint2(pack_bf16x2(a[v].x, a[v].y), pack_bf16x2(a[v].z, a[v].w));
-    else
-      *reinterpret_cast<float4*>(static_cast<float*>(p.out) + o) = a[v];
-  }
-}
-
 template <class C, int ACT>
 __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   constexpr int BM = C::BM, BN = C::BN, WM = C::WM, WN = C::WN, MI = C::MI, NI = C::NI;
@@ -323,51 +96,12 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
 
   // ---- which (split, expert M-tile, N-tile): workgroup ids are made
   // XCD-contiguous, then mapped by tile_of (or its precomputed table).
-  const int nn = p.n_ntiles;
-  const int per_split = *p.n_tiles * nn;
   const int64_t kbytes = FP8 ? p.Kred : p.Kred * 2;  // bytes per operand row
   const int nk_all = static_cast<int>(kbytes / SB);
-  int L, split, n_splits = p.splits;
-  int tail = -1;  // tail-split workgroup: its pair index in p.tail_part
-  if (MODE == Mode::kGemm2 && p.tail_split > 1) {
-    const TailPlan t = tail_plan(per_split, static_cast<int>(blockIdx.x) % kNumXcd, p.tail_split,
-                                 p.tail_slots, nk_all);
-    const int i = static_cast<int>(blockIdx.x) / kNumXcd;  // dispatch position within the XCD
-    if (i < t.full) {
-      L = t.base + i;
-      split = 0;
-      n_splits = 1;
-    } else {
-      const int j = i - t.full;
-      if (j >= t.tl * t.S) return;
-      L = t.base + t.full + j / t.S;
-      split = j % t.S;
-      n_splits = t.S;
-      tail = tail_offset(per_split, static_cast<int>(blockIdx.x) % kNumXcd, p.tail_split, p.tail_slots,
-                         nk_all) + j;
-      if (tail >= p.tail_pairs) return;  // the host sizes tail_part for every pair
-    }
-  } else {
-    const int live = per_split * p.splits;
-    if (static_cast<int>(blockIdx.x) >= live) return;
-    L = xcd_remap(blockIdx.x, live);
-    split = L / per_split;
-    L -= split * per_split;
-  }
-  int e, nt, row_beg, row_end;
-  if (p.tile_lut) {
-    const int4 v = p.tile_lut[L];
-    e = v.x;
-    nt = v.y;
-    row_beg = v.z;
-    row_end = v.w;
-  } else {
-    const Tile t = tile_of<BM>(p, L, lane);
-    e = t.e;
-    nt = t.nt;
-    row_beg = t.row_beg;
-    row_end = t.row_end;
-  }
+  Work w;
+  if (!locate<BM, MODE>(p, nk_all, lane, w)) return;
+  const int split = w.split, n_splits = w.n_splits, tail = w.tail;
+  const int e = w.e, nt = w.nt, row_beg = w.row_beg, row_end = w.row_end;
 
   // An expert's last M-tile is often nearly empty (Mixtral M=4096: ~1024 +- 30
   // slots per expert, so about half the experts add a fifth 256-row tile of a
@@ -821,76 +555,15 @@ __global__ __launch_bounds__(C::NT) void gemm_prefill_kernel(GemmParams p) {
   }
 }
 
-// Workgroup slots of one XCD for a configuration's kernel (workgroups per CU
-// x CUs per XCD); 0 when the runtime cannot say (the tail split is then off).
 template <class C>
-int xcd_slots() {
-  static const int slots = [] {
-    int dev = 0, cus = 0, occ = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, gemm_prefill_kernel<C, kActSilu>, C::NT, 0) != hipSuccess) {
-      (void)hipGetLastError();  // not left for the next launch's check to report
-      return 0;
-    }
-    return (cus % kNumXcd == 0 && occ > 0) ? occ * (cus / kNumXcd) : 0;
-  }();
-  return slots;
-}
-
-// Partials the tail split of a GEMM2 launch may need: at most one round of
-// an XCD's slots per XCD, and at most kTailMaxSplit per live tile.
-template <class C>
-int64_t tail_pairs_for(int64_t max_tiles, int64_t Nout) {
-  const int slots = xcd_slots<C>();
-  if (slots <= 0) return 0;
-  const int64_t nn = (Nout + C::BN - 1) / C::BN;
-  return std::min<int64_t>(static_cast<int64_t>(kNumXcd) * slots, max_tiles * nn * kTailMaxSplit);
-}
-
-template <class C>
-int launch(const GemmParams& p0, hipStream_t s) {
-  GemmParams p = p0;
-  const int64_t ncols = C::MODE == Mode::kGemm1Silu ? p.N_act : p.Nout;
-  const int per_tile = C::MODE == Mode::kGemm1Silu ? C::BN / 2 : C::BN;
-  p.n_ntiles = static_cast<int>((ncols + per_tile - 1) / per_tile);
-  if (p.group_tiles <= 0) p.group_tiles = kGroupTiles;
-  if (p.splits < 1) p.splits = 1;
-  int64_t grid = static_cast<int64_t>(p.max_tiles) * p.n_ntiles * p.splits;
-  if (C::MODE == Mode::kGemm2 && p.tail_split > 1) {
-    const int slots = xcd_slots<C>();
-    const int64_t pairs = tail_pairs_for<C>(p.max_tiles, p.Nout);
-    p.tail_pairs = static_cast<int64_t>(p.tail_bytes / (static_cast<size_t>(C::BM) * C::BN * sizeof(float)));
-    if (slots <= 0 || !p.tail_part || pairs <= 0 || p.tail_pairs < pairs || p.splits != 1) {
-      p.tail_split = 0;  // whole tiles only
-    } else {
-      p.tail_slots = slots;
-      const int64_t per_xcd = (static_cast<int64_t>(p.max_tiles) * p.n_ntiles + kNumXcd - 1) / kNumXcd;
-      grid = kNumXcd * (per_xcd + slots);  // whole tiles + one round of tail workgroups per XCD
-    }
-  }
-  if (grid <= 0) return FMOE_OK;
-  if (grid > 0x7fffffff) return fmoe_host::fail(FMOE_ERR_UNSUPPORTED, "prefill grid too large");
+int launch(const GemmParams& p, hipStream_t s) {
   if (C::FP8 && p.Kred / 128 > C::KST)
     return fmoe_host::fail(FMOE_ERR_UNSUPPORTED, "prefill fp8: reduction dim %lld is not supported",
                            static_cast<long long>(p.Kred));
-  if (p.tile_lut) {
-    const int64_t lut_n = static_cast<int64_t>(p.max_tiles) * p.n_ntiles;
-    tile_lut_kernel<C::BM><<<dim3(static_cast<unsigned>((lut_n + 3) / 4)), dim3(256), 0, s>>>(p);
-  }
-  const dim3 g(static_cast<unsigned>(grid)), b(C::NT);
-  if (C::MODE == Mode::kGemm2 || p.act == kActSilu)
-    gemm_prefill_kernel<C, kActSilu><<<g, b, 0, s>>>(p);
-  else if (p.act == kActGelu)
-    gemm_prefill_kernel<C, kActGelu><<<g, b, 0, s>>>(p);
-  else
-    gemm_prefill_kernel<C, kActSwiglu><<<g, b, 0, s>>>(p);
-  if (C::MODE == Mode::kGemm2 && p.tail_split > 1) {
-    const int stages = static_cast<int>((C::FP8 ? p.Kred : 2 * p.Kred) / C::SB);
-    tail_fold_kernel<C::BM, C::BN>
-        <<<dim3(static_cast<unsigned>(kNumXcd * p.tail_slots * (C::BM / kFoldRows))), dim3(256), 0, s>>>(p, stages);
-  }
-  return fmoe_host::check_launch("gemm_prefill");
+  Kernel k = gemm_prefill_kernel<C, kActSilu>;
+  if (C::MODE == Mode::kGemm1Silu && p.act == kActGelu) k = gemm_prefill_kernel<C, kActGelu>;
+  if (C::MODE == Mode::kGemm1Silu && p.act == kActSwiglu) k = gemm_prefill_kernel<C, kActSwiglu>;
+  return launch_tiles<C>(p, s, static_cast<int>((C::FP8 ? p.Kred : 2 * p.Kred) / C::SB), k);
 }
 
 }  // namespace prefill
@@ -942,7 +615,8 @@ int launch_prefill(WType wt, Mode mode, int bm, const GemmParams& p, hipStream_t
 size_t prefill_tail_bytes(WType wt, int bm, int64_t max_tiles, int64_t Nout) {
   using namespace prefill;
 #define T(BM, BN, WMS, WNS, NB, F8) \
-  static_cast<size_t>(tail_pairs_for<Cfg<BM, BN, WMS, WNS, NB, F8, Mode::kGemm2>>(max_tiles, Nout)) * BM * BN * 4
+  static_cast<size_t>(tail_pairs_for<Cfg<BM, BN, WMS, WNS, NB, F8, Mode::kGemm2>>( \
+      gemm_prefill_kernel<Cfg<BM, BN, WMS, WNS, NB, F8, Mode::kGemm2>, kActSilu>, max_tiles, Nout)) * BM * BN * 4
   if (wt != WType::kFp8) {
     if (wt != WType::kBf16) return 0;
     if (bm == 256) return T(256, 256, 4, 2, 2, false);
