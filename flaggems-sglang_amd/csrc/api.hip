@@ -8,6 +8,7 @@ namespace fmoe {
 int launch_prefill(WType wt, Mode mode, int bm, const GemmParams& p, hipStream_t s);
 size_t prefill_tail_bytes(WType wt, int bm, int64_t max_tiles, int64_t Nout);
 int launch_w4(Mode mode, const GemmParams& p, hipStream_t s);
+int launch_mx(Mode mode, int bm, const GemmParams& p, hipStream_t s);
 size_t w4_tail_bytes(int64_t max_tiles, int64_t Nout);
 int rows_for_int4(const void* x, int64_t M, int64_t K, void* xp, float* xs, hipStream_t s);
 int decode_int4_row_split(int64_t max_tiles);
@@ -159,9 +160,29 @@ int choose_block_m(int wtype, int64_t M, int k, int E, int path) {
 // fp8 160-row GEMM2's 384 columns make fewer tiles than this says).
 int prefill_bn(int wtype, int bm) { return wtype == FMOE_W_BF16 && bm <= 64 ? 128 : kPrefillBN; }
 
-// The 160-row fp8 tile stages the weight scales of at most 64 reduction
-// blocks (K, N <= 8192); larger fp8 layers take 128-row tiles.
-int fit_block_m(int wtype, int bm, int64_t K, int64_t N) {
+// Tile height of MXFP4 batches (path 0): 16 = the streaming kernels, else the
+// prefill kernels that convert in registers.  These stream 256 weight rows per
+// workgroup, so a layer whose GEMM1 makes fewer workgroups than two per CU
+// keeps the streaming kernels longer; tiled weights, which those read faster,
+// somewhat longer too.  Streaming / prefill in us a call, row-major (tiled):
+// Mixtral M=4 (1 slot per expert) 165 / 149 (128 / 139), M=16 (4) 238 / 196 (186 /
+// 180), M=64 (16) 368 / 230 (286 / 218); TP-8 (N = 1792) M=64 65 / 77 (55 / 77),
+// M=100 (25) 80 / 78 (68 / 78).
+int mx_block_m(int wtype, int64_t M, int k, int E, int64_t N) {
+  const int64_t slots = M * k, used = slots < E ? slots : E;
+  const bool wide = used * (N / 128) >= 448;
+  const int mean_stream = wide ? (is_tiled(wtype) ? 3 : 1) : (is_tiled(wtype) ? 36 : 24);
+  if (mean_at_most(slots, E, mean_stream)) return kDecodeBM;
+  const int64_t mean = slots / E;
+  return mean <= 22 ? 32 : (mean <= 48 ? 64 : 128);
+}
+
+// The height for a K x N layer.  The 160-row fp8 tile stages the weight scales
+// of at most 64 reduction blocks (K, N <= 8192); larger fp8 layers take 128-row
+// tiles.
+int layer_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {
+  if (is_mx(wtype) && path == 0) return mx_block_m(wtype, M, k, E, N);
+  const int bm = choose_block_m(wtype, M, k, E, path);
   return wtype == FMOE_W_FP8 && bm == 160 && (K > 8192 || N > 8192) ? 128 : bm;
 }
 
@@ -172,7 +193,7 @@ extern "C" int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path)
 }
 
 extern "C" int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {
-  return fit_block_m(wtype, choose_block_m(wtype, M, k, E, path), K, N);
+  return layer_block_m(wtype, M, k, E, path, K, N);
 }
 
 extern "C" int fmoe_gemm2_splits(int wtype, int64_t K, int64_t N, const fmoe_routing* r, int path) {
@@ -184,7 +205,17 @@ extern "C" int fmoe_gemm2_splits(int wtype, int64_t K, int64_t N, const fmoe_rou
     // >= 6 waves of one workgroup per CU, so the last wave's tail stays small.
     // Partials are summed by moe_sum.
     const int64_t slots = r->n_tokens * r->top_k;
-    const int64_t tiles = (slots + r->block_m - 1) / r->block_m;
+    int64_t tiles = (slots + r->block_m - 1) / r->block_m;
+    if (is_mx(wtype)) {
+      // MXFP4 (a stage is 128 elements, up to two workgroups per CU): fill the
+      // chip once, each part at least 8 stages
+      const int64_t used = slots < r->n_experts ? slots : r->n_experts;
+      if (tiles < used) tiles = used;
+      const int64_t w = tiles * ((K + kPrefillBN - 1) / kPrefillBN);
+      int64_t sp = (r->block_m <= 64 ? 512 : 256) / (w > 0 ? w : 1);
+      if (sp > N / 128 / 8) sp = N / 128 / 8;
+      return static_cast<int>(sp < 1 ? 1 : (sp > 8 ? 8 : sp));
+    }
     const int64_t wgs = tiles * ((K + kPrefillBN - 1) / kPrefillBN);
     if (wgs >= kPrefillNoSplitWgs) return 1;
     const int64_t stage_elems = wtype == FMOE_W_BF16 ? 32 : 128;
@@ -286,8 +317,8 @@ int gemm1_impl(int wtype, const void* x, const float* x_scale, const void* w13,
     return fail(FMOE_ERR_INVALID, "gemm1: int4 needs w13_scale and w13_zero");
   if (is_mx(wtype) && !w13_scale)
     return fail(FMOE_ERR_INVALID, "gemm1: mxfp4 needs w13_scale (e8m0 block scales)");
-  if (decode_only(wtype) && !is_decode(r))
-    return fail(FMOE_ERR_UNSUPPORTED, "gemm1: int4 / mxfp4 weights need block_m=16 routing");
+  if (is_int4(wtype) && !is_decode(r))
+    return fail(FMOE_ERR_UNSUPPORTED, "gemm1: int4 weights need block_m=16 routing");
   if ((path == 1 && is_decode(r)) || (path == 2 && !is_decode(r)))
     return fail(FMOE_ERR_INVALID, "gemm1: path %d does not match block_m=%d", path, r->block_m);
   GemmParams p = base_params(r);
@@ -315,6 +346,7 @@ int gemm1_impl(int wtype, const void* x, const float* x_scale, const void* w13,
   p.act_qs = act_qs;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (is_decode(r)) return launch_decode(to_wt(wtype), Mode::kGemm1Silu, p, s);
+  if (is_mx(wtype)) return launch_mx(Mode::kGemm1Silu, r->block_m, p, s);
   return launch_prefill(to_wt(wtype), Mode::kGemm1Silu, r->block_m, p, s);
 }
 }  // namespace
@@ -357,8 +389,8 @@ int gemm2_impl(int wtype, const void* act, const float* act_scale, const void* w
     return fail(FMOE_ERR_INVALID, "gemm2: int4 needs w2_scale and w2_zero");
   if (is_mx(wtype) && !w2_scale)
     return fail(FMOE_ERR_INVALID, "gemm2: mxfp4 needs w2_scale (e8m0 block scales)");
-  if (decode_only(wtype) && !is_decode(r))
-    return fail(FMOE_ERR_UNSUPPORTED, "gemm2: int4 / mxfp4 weights need block_m=16 routing");
+  if (is_int4(wtype) && !is_decode(r))
+    return fail(FMOE_ERR_UNSUPPORTED, "gemm2: int4 weights need block_m=16 routing");
   if ((path == 1 && is_decode(r)) || (path == 2 && !is_decode(r)))
     return fail(FMOE_ERR_INVALID, "gemm2: path %d does not match block_m=%d", path, r->block_m);
   if (splits < 1 || splits > 64)
@@ -389,6 +421,7 @@ int gemm2_impl(int wtype, const void* act, const float* act_scale, const void* w
   p.tail_bytes = tail_bytes;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (is_decode(r)) return launch_decode(to_wt(wtype), Mode::kGemm2, p, s);
+  if (is_mx(wtype)) return launch_mx(Mode::kGemm2, r->block_m, p, s);
   return launch_prefill(to_wt(wtype), Mode::kGemm2, r->block_m, p, s);
 }
 }  // namespace
@@ -485,7 +518,7 @@ FusedLayout layout(const fmoe_fused_args* a) {
   // expert parallel: a local expert's share of the slots follows from the
   // global expert count (the other ranks' experts take the rest)
   const int experts = a->expert_map && a->n_global > a->E ? a->n_global : a->E;
-  L.bm = fit_block_m(a->wtype, choose_block_m(a->wtype, a->M, a->top_k, experts, a->path), a->K, a->N);
+  L.bm = layer_block_m(a->wtype, a->M, a->top_k, experts, a->path, a->K, a->N);
   L.w4 = w4_route(a);
   if (L.w4) L.bm = kW4BM;
   L.max_tiles = fmoe_max_tiles(slots, a->E);
@@ -540,7 +573,7 @@ FusedLayout layout(const fmoe_fused_args* a) {
   L.acts = take(fp8 || L.w4 ? 4 * slots * (a->N / 128) : 0);
   // prefill with one split: bf16 rows (see fused path); otherwise fp32 planes
   // (the int4 prefill kernels' rows are fp32, as the streaming kernels' are)
-  L.y_bf16 = L.bm != kDecodeBM && !L.w4 && L.splits == 1 && !mean_at_most(slots, a->E, kFp32RowsMean);
+  L.y_bf16 = L.bm != kDecodeBM && !L.w4 && !is_mx(a->wtype) && L.splits == 1 && !mean_at_most(slots, a->E, kFp32RowsMean);
   L.y = take((L.y_bf16 ? 2 : 4) * static_cast<size_t>(L.splits) * slots * a->K);
   // prefill: tile table, shared by the two GEMM launches (stream order)
   const int bn = prefill_bn(a->wtype, L.bm);

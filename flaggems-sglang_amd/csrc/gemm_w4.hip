@@ -21,9 +21,10 @@
 namespace fmoe {
 namespace prefill {
 
-template <int BM_, int WAVES_M_, int WAVES_N_, int NBUF_, Mode MODE_>
+template <int BM_, int WAVES_M_, int WAVES_N_, int NBUF_, bool MX_, Mode MODE_>
 struct W4Cfg {
   static constexpr int BM = BM_, BN = 256, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, NBUF = NBUF_;
+  static constexpr bool MX = MX_;
   static constexpr Mode MODE = MODE_;
   static constexpr int NW = WAVES_M * WAVES_N, NT = NW * 64;
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / 16, NI = WN / 16;
@@ -32,13 +33,17 @@ struct W4Cfg {
   static constexpr int A_UNITS = BM / 16 * 4, B_UNITS = BN / 16, UNITS = A_UNITS + B_UNITS;
   static constexpr int UPW = (UNITS + NW - 1) / NW;
   static constexpr int STAGE = UNITS * kUnit;
-  // small loads of a stage, one wave each (the last waves): scales of 128
-  // weight rows (2), zeros (1), row sums of 64 slots
-  static constexpr int AUX = 3 + (BM + 63) / 64;
+  // small loads of a stage, one wave each (the last waves).  int4: scales of
+  // 128 weight rows (2), zeros (1), row sums of 64 slots; MXFP4: the four
+  // scale bytes of 64 weight rows (4)
+  static constexpr int AUX = MX ? BN / 64 : 3 + (BM + 63) / 64;
+  // MXFP4 scale slots hold 16 bytes (four stages) per weight row
+  static constexpr int AUX_LDS = MX ? 2 * BN * 16 : NBUF * (BN * 2 + BN / 2 + BM * 4);
+  static_assert(!MX || NBUF <= 4, "two scale slots cover the ring");
   static_assert(UNITS % NW == 0, "every wave issues UPW units");
   static_assert(AUX <= NW, "one small load per wave");
   static_assert((MODE == Mode::kGemm1Silu ? NI / 2 : NI) % 2 == 0, "weight blocks in pairs");
-  static_assert(NBUF * (STAGE + BN * 2 + BN / 2 + BM * 4) <= 160 * 1024, "LDS budget");
+  static_assert(NBUF * STAGE + AUX_LDS <= 160 * 1024, "LDS budget");
 };
 
 // x rows in the nibble order, and their group sums: one thread per 8 elements,
@@ -69,9 +74,11 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
   constexpr int BM = C::BM, BN = C::BN, WM = C::WM, WN = C::WN, MI = C::MI, NI = C::NI, NW = C::NW, NBUF = C::NBUF;
   constexpr Mode MODE = C::MODE;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NBUF][C::STAGE];
-  __shared__ __attribute__((aligned(256))) uint16_t sc_lds[NBUF][BN];
-  __shared__ __attribute__((aligned(256))) uint32_t zr_lds[NBUF][BN / 8];
-  __shared__ __attribute__((aligned(256))) float xs_lds[NBUF][BM];
+  // int4: fp16 scales, u4 zeros, row sums; MXFP4: scale bytes per weight row
+  __shared__ __attribute__((aligned(256))) uint16_t sc_lds[NBUF][C::MX ? 1 : BN];
+  __shared__ __attribute__((aligned(256))) uint32_t zr_lds[NBUF][C::MX ? 1 : BN / 8];
+  __shared__ __attribute__((aligned(256))) float xs_lds[NBUF][C::MX ? 1 : BM];
+  __shared__ __attribute__((aligned(256))) uint32_t mx_lds[C::MX ? 2 * BN * 4 : 1];
 
   const int tid = threadIdx.x, lane = tid % kWave, g = lane >> 4, r16 = lane & 15;
   const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -135,7 +142,12 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
   uint8_t* aux_dst = nullptr;
   int aux_slot = 0;
   bool aux_lane = aux < C::AUX;
-  if (aux < 2) {  // scales of tile columns 128 aux + 2 lane, + 1
+  if constexpr (C::MX) {
+    if (aux < C::AUX) {  // scale bytes of LDS weight rows 64 aux + lane
+      const int row = 64 * aux + lane;
+      aux_src = p.b_mxscale + (static_cast<int64_t>(e) * p.Nout + w_row(tile_row<true>(row / 16, row % 16))) * (4 * groups);
+    }
+  } else if (aux < 2) {  // scales of tile columns 128 aux + 2 lane, + 1
     const int tc = 128 * aux + 2 * lane;
     aux_src = reinterpret_cast<const uint8_t*>(p.b_gscale + (static_cast<int64_t>(e) * groups + k0) * p.Nout + w_row(tc));
     aux_step = 2 * p.Nout;
@@ -156,11 +168,26 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
     aux_slot = BM * 4;
     aux_lane = r < BM;
   }
-  const int per = C::UPW + (aux < C::AUX ? 1 : 0);
+  // MXFP4 scales: a load per row and stage touches a line per lane, so where
+  // a row's scale bytes divide into 16-byte pieces they come for four stages
+  // at once (Mixtral M=33 GEMM1 146 -> 110 us without the per-stage loads)
+  const bool mx_quads = groups % 4 == 0;
+  // loads per stage that every wait may count on (the scale loads of four
+  // stages come on top: a wait that sees one waits for that one too)
+  const int per = C::UPW + (aux < C::AUX && !(C::MX && mx_quads) ? 1 : 0);
   auto issue_unit = [&](int kt, int i) {
     dma16(src[i] + static_cast<int64_t>(kt) * step_bytes[i], lds[kt % NBUF] + (NW * i + wid) * kUnit);
   };
   auto issue_aux = [&](int kt) {
+    if constexpr (C::MX) {
+      if (aux >= C::AUX) return;
+      const int k = k0 + kt;
+      if (!mx_quads)
+        dma4(reinterpret_cast<const float*>(aux_src + 4 * k), reinterpret_cast<float*>(&mx_lds[(kt % NBUF) * BN + 64 * aux]));
+      else if (kt == 0 || k % 4 == 0)
+        dma16(aux_src + 16 * (k / 4), reinterpret_cast<uint8_t*>(&mx_lds[(k / 4 % 2) * (4 * BN) + 256 * aux]));
+      return;
+    }
     if (aux < C::AUX)
       if (aux_lane)
         dma4(reinterpret_cast<const float*>(aux_src + kt * aux_step),
@@ -199,14 +226,23 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
   const int bo = p.b_tiled ? 16 * lane : 16 * (4 * r16 + (g ^ (r16 >> 1 & 3)));
   bf16x8_t fa[2][MI];
   i32x4_t bq[NI];
+  uint32_t mx[NI];  // MXFP4: the scale bytes of the lane's row of each block
   auto read_a = [&](int slot, int s, int q) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
       fa[q][i] = __builtin_bit_cast(bf16x8_t, lds16(lds[slot] + (wm * MI + i) * 4 * kUnit + fo[s]));
   };
-  auto read_b = [&](int slot) {
+  auto read_b = [&](int kt) {
+    const int slot = kt % NBUF;
 #pragma unroll
     for (int j = 0; j < NI; ++j) bq[j] = lds16(lds[slot] + (C::A_UNITS + wn * NI + j) * kUnit + bo);
+    if constexpr (C::MX) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const int row = (wn * NI + j) * 16 + r16, k = k0 + kt;
+        mx[j] = mx_lds[mx_quads ? (k / 4 % 2) * (4 * BN) + 4 * row + k % 4 : slot * BN + row];
+      }
+    }
   };
   // the two constants in registers, so that and + or are one v_and_or_b32
   uint32_t nib_mask, nib_one, nib_f32;
@@ -238,7 +274,66 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
     // One stage: the fragments of step s + 1 are read during step s; before
     // the last step the slot's reads are over, and one wait and one barrier
     // publish the next stage and free the slot (as gemm_prefill_kernel).
-    auto stage = [&](int kt, auto more, auto dma) {
+    // MXFP4: e2m1 -> bf16 with the block's scale folded in (exact), straight
+    // into the accumulators
+    auto stage_mx = [&](int kt, auto more, auto dma) {
+      constexpr bool MORE = decltype(more)::value, DMA = decltype(dma)::value;
+      const int slot = kt % NBUF, next = (kt + 1) % NBUF;
+      float sc[NI];  // the lane's 32 elements of the group are scale block g
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const uint32_t ex = __builtin_amdgcn_ubfe(mx[j], 8 * g, 8);
+        sc[j] = ex == 0 ? 0x1p-127f : (ex == 255 ? __builtin_nanf("") : __uint_as_float(ex << 23));
+      }
+      auto cvt = [&](int j, int s) {
+        const uint32_t v = static_cast<uint32_t>(bq[j][s]);
+        i32x4_t o;
+        o[0] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc[j], 0));
+        o[1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc[j], 1));
+        o[2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc[j], 2));
+        o[3] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc[j], 3));
+        return __builtin_bit_cast(bf16x8_t, o);
+      };
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        read_a(slot, s + 1, (s + 1) & 1);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const bf16x8_t fb = cvt(j, s);
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb, fa[s & 1][i], acc[i][j], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      bf16x8_t fb[NI];
+#pragma unroll
+      for (int j = 0; j < NI; ++j) fb[j] = cvt(j, 3);
+      if constexpr (MORE) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads have left the slot
+        if constexpr (DMA)
+          wait_full(Ring2{});
+        else
+          wait_stage(min(NBUF - 2, nk - 2 - kt));
+        read_a(next, 0, 0);
+        read_b(kt + 1);
+      }
+      if constexpr (DMA) issue_aux(kt + NBUF);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (DMA) {
+#pragma unroll
+          for (int u = 0; u < C::UPW; ++u)
+            if (u * NI / C::UPW == j) issue_unit(kt + NBUF, u);
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[1][i], acc[i][j], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto stage_int4 = [&](int kt, auto more, auto dma) {
       constexpr bool MORE = decltype(more)::value, DMA = decltype(dma)::value;
       const int slot = kt % NBUF, next = (kt + 1) % NBUF;
       f32x4_t t[MI][NI];
@@ -279,7 +374,7 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
         else
           wait_stage(min(NBUF - 2, nk - 2 - kt));
         read_a(next, 0, 0);
-        read_b(next);
+        read_b(kt + 1);
       }
       if constexpr (DMA) issue_aux(kt + NBUF);
       // the last step's products of block column j, then the fold of column j - 1
@@ -314,6 +409,12 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
             acc[i][j - 1][r] = __builtin_fmaf(sv[r], __builtin_fmaf(-zv[r], xs[i], t[i][j - 1][r]), acc[i][j - 1][r]);
       }
     };
+    auto stage = [&](int kt, auto more, auto dma) {
+      if constexpr (C::MX)
+        stage_mx(kt, more, dma);
+      else
+        stage_int4(kt, more, dma);
+    };
     int kt = 0;
     for (; kt + NBUF < nk; ++kt) stage(kt, T{}, T{});
     for (; kt + 1 < nk; ++kt) stage(kt, T{}, F{});
@@ -331,7 +432,39 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
   }
 #pragma unroll
   for (int i = 0; i < MI; ++i) asm volatile("" ::"v"(gv[i]));
-  if constexpr (MODE == Mode::kGemm1Silu) {
+  if constexpr (MODE == Mode::kGemm1Silu && C::MX) {
+    uint16_t* act = static_cast<uint16_t*>(p.out);
+    const int64_t c0 = static_cast<int64_t>(nt) * (BN / 2) + wn * (WN / 2);
+    float gb[NI / 2][4], ub[NI / 2][4];
+#pragma unroll
+    for (int j = 0; j < NI / 2; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        gemm1_bias<ACT>(p, e, c0 + tile_col<true>(j, lane) + c, gb[j][c], ub[j][c]);
+        asm volatile("" ::"v"(gb[j][c]), "v"(ub[j][c]));
+      }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int s = row_beg + wm * WM + i * 16 + r16;
+      if (s >= row_end) continue;
+#pragma unroll
+      for (int j = 0; j < NI / 2; j += 2) {
+        uint4 o;
+        uint32_t* ow = reinterpret_cast<uint32_t*>(&o);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          float a[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int jj = j + h / 2, c = 2 * (h % 2) + u;
+            a[u] = gemm1_act<ACT>(p, acc[i][jj][c], acc[i][jj + NI / 2][c], gb[jj][c], ub[jj][c], gv[i]);
+          }
+          ow[h] = pack_bf16x2(a[0], a[1]);
+        }
+        *reinterpret_cast<uint4*>(act + static_cast<int64_t>(s) * p.N_act + c0 + tile_col<true>(j, lane)) = o;
+      }
+    }
+  } else if constexpr (MODE == Mode::kGemm1Silu) {
     // bf16 activations in the nibble order, and their group sums (of the
     // rounded values): lane, the row's 4 lanes, then the waves through LDS
     __syncthreads();
@@ -413,15 +546,39 @@ __global__ __launch_bounds__(C::NT) void gemm_w4_kernel(GemmParams p) {
 // 128-row tiles, 2x4 waves, 3-deep ring of 48 KiB stages.
 int launch_w4(Mode mode, const GemmParams& p, hipStream_t s) {
   using namespace prefill;
-  using C1 = W4Cfg<128, 2, 4, 3, Mode::kGemm1Silu>;
-  using C2 = W4Cfg<128, 2, 4, 3, Mode::kGemm2>;
+  using C1 = W4Cfg<128, 2, 4, 3, false, Mode::kGemm1Silu>;
+  using C2 = W4Cfg<128, 2, 4, 3, false, Mode::kGemm2>;
   const int groups = static_cast<int>(p.Kred / 128);
   if (mode == Mode::kGemm2) return launch_tiles<C2>(p, s, groups, gemm_w4_kernel<C2, kActSilu>);
   return launch_tiles<C1>(p, s, groups, p.act == kActGelu ? gemm_w4_kernel<C1, kActGelu> : gemm_w4_kernel<C1, kActSilu>);
 }
 
+// MXFP4: 128 rows as int4; 64 and 32 rows with 2- and 3-deep rings, two
+// workgroups per CU (72 and 80 KiB of LDS).  Mixtral, 32 rows, 2x4 / 1x4 waves:
+// M=33 200 / 209 us a call; a 4-deep ring (one workgroup per CU) 224; 64 rows,
+// 2-deep / 4-deep: M=100 230 / 287.
+int launch_mx(Mode mode, int bm, const GemmParams& p, hipStream_t s) {
+  using namespace prefill;
+  const int groups = static_cast<int>(p.Kred / 128);
+#define G1(BM, WMS, WNS, NB, ACT) gemm_w4_kernel<W4Cfg<BM, WMS, WNS, NB, true, Mode::kGemm1Silu>, ACT>
+#define L(BM, WMS, WNS, NB)                                                                                  \
+  (mode == Mode::kGemm2                                                                                      \
+       ? launch_tiles<W4Cfg<BM, WMS, WNS, NB, true, Mode::kGemm2>>(                                          \
+             p, s, groups, gemm_w4_kernel<W4Cfg<BM, WMS, WNS, NB, true, Mode::kGemm2>, kActSilu>)            \
+       : launch_tiles<W4Cfg<BM, WMS, WNS, NB, true, Mode::kGemm1Silu>>(                                      \
+             p, s, groups, p.act == kActSwiglu ? G1(BM, WMS, WNS, NB, kActSwiglu)                            \
+                                               : (p.act == kActGelu ? G1(BM, WMS, WNS, NB, kActGelu)         \
+                                                                    : G1(BM, WMS, WNS, NB, kActSilu))))
+  if (bm == 128) return L(128, 2, 4, 3);
+  if (bm == 64) return L(64, 2, 4, 2);
+  if (bm == 32) return L(32, 2, 4, 3);
+#undef L
+#undef G1
+  return fmoe_host::fail(FMOE_ERR_UNSUPPORTED, "mxfp4 prefill: block_m=%d is not supported", bm);
+}
+
 size_t w4_tail_bytes(int64_t max_tiles, int64_t Nout) {
-  using C = prefill::W4Cfg<128, 2, 4, 3, Mode::kGemm2>;
+  using C = prefill::W4Cfg<128, 2, 4, 3, false, Mode::kGemm2>;
   return static_cast<size_t>(prefill::tail_pairs_for<C>(prefill::gemm_w4_kernel<C, kActSilu>, max_tiles, Nout)) *
          C::BM * C::BN * 4;
 }

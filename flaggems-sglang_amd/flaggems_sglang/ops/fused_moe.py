@@ -518,7 +518,7 @@ def triton_kernel_fused_experts_with_bias(
         assert tuple(s13.shape) == (E, N2, Kh // 32) and tuple(s2t.shape) == (E, Kh, w2t.shape[2] * 2 // 32), \
             "mxfp4 scale shapes do not match the weights"
         require_cuda(s13, s2t)
-    bm = lib().fmoe_choose_block_m(wtype, M, k, E, 0)
+    bm = _block_m(wtype, M, k, E, 0, Kh, w13.shape[1] // 2)
     offs_raw, offs_pad, tile_map, n_tiles = _expt_data_for(routing_data, M * k, bm)
     topk_indx = gather_indx.src_indx.to(torch.int32).contiguous()
     gate_indx = gather_indx.dst_indx.to(torch.int32).contiguous()
@@ -754,8 +754,12 @@ def fused_moe_flagos(obj, layer: torch.nn.Module, dispatch_output):
         if _is_triton_routing(topk_output):
             routing_data, gather_indx, scatter_indx = topk_output
         else:
+            ids = topk_output.topk_ids
+            # the tile map for the height the GEMMs will use
+            bm = _block_m(W_MXFP4 if quant else W_BF16, ids.shape[0], ids.shape[1], cfg.num_experts, 0,
+                          hidden_states.shape[-1], w13.shape[1] // 2)
             routing_data, gather_indx, scatter_indx = _standard_topk_to_triton_kernels(
-                topk_output.topk_weights, topk_output.topk_ids, cfg.num_experts)
+                topk_output.topk_weights, ids, cfg.num_experts, block_m=bm)
         out = triton_kernel_fused_experts_with_bias(
             hidden_states, w13.transpose(-1, -2), pcg13, b13, w2.transpose(-1, -2), pcg2, b2,
             routing_data, gather_indx, None if no_combine else scatter_indx, activation=activation,

@@ -1,0 +1,99 @@
+"""MXFP4 on the prefill kernels that convert in registers: every tile height,
+row-major and tiled weights, scale bytes in 16-byte pieces (reductions of a
+multiple of four groups) and one by one, split reductions, SwiGLU with biases,
+scale bytes 0 and 255, against the oracle and the streaming kernels."""
+
+import pytest
+import torch
+
+from flaggems_sglang import _lib
+from flaggems_sglang import quant as Q
+from oracle import fused_moe_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _ids(counts, k=2):
+    flat = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    return flat.view(k, -1).t().contiguous().to(torch.int32)
+
+
+def _rel(a, b):
+    # exact weights on both sides: rows differ by bf16 rounding flips only
+    return float(((a - b).norm(dim=1) / b.norm(dim=1).clamp_min(1e-20)).max())
+
+
+def _problem(counts, K, N, seed=0):
+    ids = _ids(counts)
+    d = O.make_inputs(ids.shape[0], K, N, len(counts), 2, wscale=0.05, seed=seed)
+    return d, ids, Q.quantize_mxfp4(d["w13"]), Q.quantize_mxfp4(d["w2"])
+
+
+COUNTS = {32: [33, 31, 1, 33, 32, 0, 30, 16], 64: [65, 1, 64, 63, 0, 33, 64, 62],
+          128: [129, 127, 1, 128, 0, 130, 100, 65]}
+
+
+@pytest.mark.parametrize("K,N", [(128, 7168), (512, 7296), (640, 7168), (384, 8192)])
+@pytest.mark.parametrize("bm", sorted(COUNTS))
+def test_heights(bm, K, N):
+    import flaggems_sglang
+
+    d, ids, (q1, s1), (q2, s2) = _problem(COUNTS[bm], K, N)
+    M = ids.shape[0]
+    assert _lib.lib().fmoe_fused_block_m(_lib.W_MXFP4, M, 2, 8, 0, K, N) == bm
+    assert _lib.lib().fmoe_fused_block_m(_lib.W_MXFP4_TILED, M, 2, 8, 0, K, N) == bm
+
+    def call(tiled, path):
+        a, b = q1.to(DEV), q2.to(DEV)
+        if tiled:
+            a, b = Q.tile_mxfp4(a), Q.tile_mxfp4(b)
+        return flaggems_sglang.fused_experts(
+            d["x"].to(DEV), a, b, d["topk_weights"].to(DEV), ids.to(DEV), path=path, use_mxfp4_w4a16=True,
+            w1_scale=s1.to(DEV), w2_scale=s2.to(DEV)).float().cpu()
+
+    out = call(False, 0)
+    assert torch.equal(out, call(True, 0))  # the layout changes addresses only
+    assert _rel(out, call(True, 2)) < 1e-2
+    ref = O.fused_experts_mxfp4(d["x"], q1, s1, q2, s2, d["topk_weights"], ids).float()
+    assert _rel(out, ref) < 1e-2
+
+
+@pytest.mark.parametrize("bm", sorted(COUNTS))
+def test_bias_swiglu(bm):
+    """The bias entry on routing of each height (narrow layers, so that the
+    routing, not the rule, picks it)."""
+    import flaggems_sglang
+    from types import SimpleNamespace
+
+    K, N = 256, 7168
+    d, ids, (q1, s1), (q2, s2) = _problem(COUNTS[bm], K, N, seed=3)
+    g = torch.Generator().manual_seed(4)
+    b13, b2 = torch.randn(8, 2 * N, generator=g) * 0.1, torch.randn(8, K, generator=g) * 0.1
+    tw = d["topk_weights"].to(DEV)
+    rd, gi, si = flaggems_sglang.ops.fused_moe._standard_topk_to_triton_kernels(tw, ids.to(DEV), 8)
+    pc = [SimpleNamespace(weight_scale=s.to(DEV).transpose(1, 2)) for s in (s1, s2)]
+    out = flaggems_sglang.triton_kernel_fused_experts_with_bias(
+        d["x"].to(DEV), q1.to(DEV).transpose(1, 2), pc[0], b13.to(DEV), q2.to(DEV).transpose(1, 2), pc[1],
+        b2.to(DEV), rd, gi, si, gemm1_alpha=1.702, gemm1_clamp_limit=7.0).float().cpu()
+    assert bm in rd.expt_data.block_pid_map
+    ref = O.fused_experts_bias(d["x"], O.mxfp4_dequant(q1, s1), b13, O.mxfp4_dequant(q2, s2), b2,
+                               d["topk_weights"], ids, alpha=1.702, limit=7.0).float()
+    assert _rel(out, ref) < 1e-2
+
+
+def test_scale_bytes_0_and_255():
+    """2^-127 and NaN scales: the outputs of the streaming kernels, NaN for NaN."""
+    import flaggems_sglang
+
+    d, ids, (q1, s1), (q2, s2) = _problem(COUNTS[32], 512, 7168, seed=5)
+    s1 = s1.clone()
+    s1[0] = 0       # expert 0: gate and up vanish
+    s2 = s2.clone()
+    s2[3, 5, 2] = 255  # expert 3: one NaN block in output column 5
+    args = (d["x"].to(DEV), q1.to(DEV), q2.to(DEV), d["topk_weights"].to(DEV), ids.to(DEV))
+    kw = dict(use_mxfp4_w4a16=True, w1_scale=s1.to(DEV), w2_scale=s2.to(DEV))
+    out = flaggems_sglang.fused_experts(*args, **kw).float().cpu()
+    dec = flaggems_sglang.fused_experts(*args, path=2, **kw).float().cpu()
+    assert torch.equal(out.isnan(), dec.isnan()) and out.isnan().any()
+    assert _rel(out.nan_to_num(0.0), dec.nan_to_num(0.0)) < 1e-2
