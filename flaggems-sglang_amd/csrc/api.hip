@@ -861,7 +861,7 @@ extern "C" int fmoe_fused_experts_noalloc(const fmoe_fused_args* a, void* stream
   fmoe_fused_args b = *a;
   // batches that the streaming kernels would also take: those need less
   if (need > FMOE_NOALLOC_SCRATCH_BYTES && a->path == 0 &&
-      (w4_route(a) || mean_at_most(a->M * a->top_k, a->E, kFp32RowsMean))) {
+      (w4_route(a) || (is_mx(a->wtype) && !dequant_prefill(a)) || mean_at_most(a->M * a->top_k, a->E, kFp32RowsMean))) {
     b.path = 2;
     need = fmoe_fused_experts_workspace_bytes(&b);
   }

@@ -484,6 +484,26 @@ def triton_kernel_fused_experts_with_bias(
     """
     logger.debug("FLAGGEMS_SGLANG FUSED_MOE_WITH_BIAS")
     assert inplace is False, "Inplace is not supported"
+    E = routing_data.n_expts_tot
+    x, w13, w2t, wtype, s13, s2t = _bias_operands(hidden_states, w1, w1_pcg, b1, w2, w2_pcg, b2, E, activation)
+    M, Kh = x.shape
+    k = routing_data.n_expts_act
+    bm = _block_m(wtype, M, k, E, 0, Kh, w13.shape[1] // 2)
+    offs_raw, offs_pad, tile_map, n_tiles = _expt_data_for(routing_data, M * k, bm)
+    topk_indx = gather_indx.src_indx.to(torch.int32).contiguous()
+    gate_indx = gather_indx.dst_indx.to(torch.int32).contiguous()
+    gate_scal = routing_data.gate_scal.float().contiguous()
+    return _run_stages(x, w13, w2t, wtype, s13, s2t, None, None, M, k, E, topk_indx,
+                       gate_indx, gate_scal, offs_raw, offs_pad, tile_map, n_tiles, bm,
+                       apply_router_weight_on_input, 1.0, combine=scatter_indx is not None,
+                       act=_lib.ACT_SWIGLU, b13=b1.float().contiguous(), b2=b2.float().contiguous(),
+                       alpha=1.0 if gemm1_alpha is None else float(gemm1_alpha),
+                       limit=0.0 if gemm1_clamp_limit is None else float(gemm1_clamp_limit))
+
+
+def _bias_operands(hidden_states, w1, w1_pcg, b1, w2, w2_pcg, b2, E, activation):
+    """Checks of the bias path; its operands in the kernels' layouts:
+    ``(x, w13, w2, wtype, w13_scale, w2_scale)``."""
     assert hidden_states.dtype == torch.bfloat16, "hidden_states must be bfloat16"
     if activation != "silu":
         raise ValueError(f"Unsupported FusedMoe activation: {activation}")
@@ -501,13 +521,10 @@ def triton_kernel_fused_experts_with_bias(
     assert hidden_states.shape[-1] == Kh, "hidden size mismatch"
     assert w2.shape[-1] == Kh, "intermediate size mismatch"
     assert b1 is not None and b2 is not None, "Bias execution requires both w13_bias and w2_bias"
-    E = routing_data.n_expts_tot
     assert tuple(b1.shape) == (E, w1.shape[2]) and tuple(b2.shape) == (E, w2.shape[2]), \
         "bias shape mismatch"
     require_cuda(hidden_states, w1, w2, b1, b2)
     x = hidden_states.contiguous()
-    M = x.shape[0]
-    k = routing_data.n_expts_act
     w13 = _as_sglang_layout(w1)
     w2t = _as_sglang_layout(w2)
     wtype, s13, s2t = _lib.W_BF16, None, None
@@ -518,17 +535,7 @@ def triton_kernel_fused_experts_with_bias(
         assert tuple(s13.shape) == (E, N2, Kh // 32) and tuple(s2t.shape) == (E, Kh, w2t.shape[2] * 2 // 32), \
             "mxfp4 scale shapes do not match the weights"
         require_cuda(s13, s2t)
-    bm = _block_m(wtype, M, k, E, 0, Kh, w13.shape[1] // 2)
-    offs_raw, offs_pad, tile_map, n_tiles = _expt_data_for(routing_data, M * k, bm)
-    topk_indx = gather_indx.src_indx.to(torch.int32).contiguous()
-    gate_indx = gather_indx.dst_indx.to(torch.int32).contiguous()
-    gate_scal = routing_data.gate_scal.float().contiguous()
-    return _run_stages(x, w13, w2t, wtype, s13, s2t, None, None, M, k, E, topk_indx,
-                       gate_indx, gate_scal, offs_raw, offs_pad, tile_map, n_tiles, bm,
-                       apply_router_weight_on_input, 1.0, combine=scatter_indx is not None,
-                       act=_lib.ACT_SWIGLU, b13=b1.float().contiguous(), b2=b2.float().contiguous(),
-                       alpha=1.0 if gemm1_alpha is None else float(gemm1_alpha),
-                       limit=0.0 if gemm1_clamp_limit is None else float(gemm1_clamp_limit))
+    return x, w13, w2t, wtype, s13, s2t
 
 
 def _pcg_scale(pcg, name):
@@ -631,13 +638,21 @@ def fused_experts(
                            a.topk_indx, a.gate_indx, a.gate_scal, a.offs_raw, a.offs_pad, a.tile_map,
                            a.n_tiles, a.block_m, apply_router_weight_on_input, 1.0, combine=False,
                            act=act, slot_order=_slot_order(topk_ids, emap))
+    return _fused_call(x, w1, w2, wtype, w1_scale, w2_scale, w1_zp, w2_zp, N, topk_weights, topk_ids,
+                       apply_router_weight_on_input, scale, path, act, emap=emap)
+
+
+def _fused_call(x, w13, w2, wtype, w13_scale, w2_scale, w13_zp, w2_zp, N, topk_weights, topk_ids, on_input,
+                scale, path, act, emap=None, b13=None, b2=None, alpha=1.0, limit=0.0):
+    """One ``fmoe_fused_experts`` call on checked operands (SGLang layouts)."""
+    M, K = x.shape
     ids = _ids_i32(topk_ids)
     tw = topk_weights.float().contiguous()
     out = torch.empty(M, K, dtype=torch.bfloat16, device=x.device)
     args = _lib.FusedArgs(
-        wtype, ptr(x), M, K, N, E, k, ptr(w1), ptr(w2), ptr(w1_scale), ptr(w2_scale), ptr(w1_zp),
-        ptr(w2_zp), 128, ptr(tw), ptr(ids), int(apply_router_weight_on_input), scale, path,
-        ptr(out), None, 0, act, None, None, 1.0, 0.0, ptr(emap), 0 if emap is None else emap.numel())
+        wtype, ptr(x), M, K, N, w13.shape[0], ids.shape[1], ptr(w13), ptr(w2), ptr(w13_scale), ptr(w2_scale),
+        ptr(w13_zp), ptr(w2_zp), 128, ptr(tw), ptr(ids), int(on_input), scale, path, ptr(out), None, 0, act,
+        ptr(b13), ptr(b2), float(alpha), float(limit), ptr(emap), 0 if emap is None else emap.numel())
     L = lib()
     nbytes = L.fmoe_fused_experts_workspace_bytes(ctypes.byref(args))
     if nbytes == 0:
@@ -689,6 +704,24 @@ def _combine_input(hidden_states):
     except Exception:
         return CombineInput(hidden_states=hidden_states)
     return StandardCombineInput(hidden_states=hidden_states)
+
+
+def _bias_mxfp4_call(hidden_states, w13, pcg13, b13, w2, pcg2, b2, topk_output, cfg, activation, on_input):
+    """The MXFP4 bias path as one C call (the stages' kernels and arithmetic,
+    without their ~20 allocations and calls from Python: Mixtral TP-8 M=16 132
+    -> 91 us a call, host-bound); None where the one call would differ: batches
+    that it dequantizes to bf16 (256 slots per expert)."""
+    E = cfg.num_experts
+    tw, ids = topk_output.topk_weights, topk_output.topk_ids
+    if ids.numel() >= 256 * E or ids.shape[1] > E or w13.shape[0] != E or w2.shape[0] != E:
+        return None
+    x, w13, w2, wtype, s13, s2 = _bias_operands(hidden_states, w13.transpose(-1, -2), pcg13, b13,
+                                                w2.transpose(-1, -2), pcg2, b2, E, activation)
+    require_cuda(tw, ids)
+    alpha, limit = getattr(cfg, "gemm1_alpha", None), getattr(cfg, "gemm1_clamp_limit", None)
+    return _fused_call(x, w13, w2, wtype, s13, s2, None, None, w13.shape[1] // 2, tw, ids, on_input, 1.0, 0,
+                       _lib.ACT_SWIGLU, b13=b13.float().contiguous(), b2=b2.float().contiguous(),
+                       alpha=1.0 if alpha is None else alpha, limit=0.0 if limit is None else limit)
 
 
 def fused_moe_flagos(obj, layer: torch.nn.Module, dispatch_output):
@@ -751,20 +784,21 @@ def fused_moe_flagos(obj, layer: torch.nn.Module, dispatch_output):
             # matmul_ogs orientation views of the SGLang-layout scales (no copy)
             pcg13 = SimpleNamespace(weight_scale=quant["w1_scale"].transpose(-1, -2))
             pcg2 = SimpleNamespace(weight_scale=quant["w2_scale"].transpose(-1, -2))
-        if _is_triton_routing(topk_output):
-            routing_data, gather_indx, scatter_indx = topk_output
-        else:
-            ids = topk_output.topk_ids
-            # the tile map for the height the GEMMs will use
-            bm = _block_m(W_MXFP4 if quant else W_BF16, ids.shape[0], ids.shape[1], cfg.num_experts, 0,
-                          hidden_states.shape[-1], w13.shape[1] // 2)
-            routing_data, gather_indx, scatter_indx = _standard_topk_to_triton_kernels(
-                topk_output.topk_weights, ids, cfg.num_experts, block_m=bm)
-        out = triton_kernel_fused_experts_with_bias(
-            hidden_states, w13.transpose(-1, -2), pcg13, b13, w2.transpose(-1, -2), pcg2, b2,
-            routing_data, gather_indx, None if no_combine else scatter_indx, activation=activation,
-            apply_router_weight_on_input=on_input, gemm1_alpha=getattr(cfg, "gemm1_alpha", None),
-            gemm1_clamp_limit=getattr(cfg, "gemm1_clamp_limit", None))
+        out = None
+        if quant and not no_combine and not _is_triton_routing(topk_output):
+            out = _bias_mxfp4_call(hidden_states, w13, pcg13, b13, w2, pcg2, b2, topk_output, cfg, activation,
+                                   on_input)
+        if out is None:
+            if _is_triton_routing(topk_output):
+                routing_data, gather_indx, scatter_indx = topk_output
+            else:
+                routing_data, gather_indx, scatter_indx = _standard_topk_to_triton_kernels(
+                    topk_output.topk_weights, topk_output.topk_ids, cfg.num_experts)
+            out = triton_kernel_fused_experts_with_bias(
+                hidden_states, w13.transpose(-1, -2), pcg13, b13, w2.transpose(-1, -2), pcg2, b2,
+                routing_data, gather_indx, None if no_combine else scatter_indx, activation=activation,
+                apply_router_weight_on_input=on_input, gemm1_alpha=getattr(cfg, "gemm1_alpha", None),
+                gemm1_clamp_limit=getattr(cfg, "gemm1_clamp_limit", None))
         if scale is not None:
             out.mul_(scale)
     elif _is_triton_routing(topk_output):

@@ -97,3 +97,40 @@ def test_scale_bytes_0_and_255():
     dec = flaggems_sglang.fused_experts(*args, path=2, **kw).float().cpu()
     assert torch.equal(out.isnan(), dec.isnan()) and out.isnan().any()
     assert _rel(out.nan_to_num(0.0), dec.nan_to_num(0.0)) < 1e-2
+
+
+@pytest.mark.parametrize("M", [0, 1, 5, 40, 300, 520])
+@pytest.mark.parametrize("on_input,rsf", [(False, None), (True, 2.5)])
+def test_hook_one_call_equals_stages(M, on_input, rsf):
+    """The hook's MXFP4 bias layer (one C call; stages again from 256 slots per
+    expert) against the bias entry on prepared routing: bit-identical."""
+    from types import SimpleNamespace
+
+    import flaggems_sglang
+    from flaggems_sglang.ops import fused_moe as F
+
+    K, N, E, k = 256, 512, 4, 2
+    d = O.make_inputs(max(M, 1), K, N, E, k, wscale=0.05)
+    x, tw, ti = (d[n][:M].to(DEV) for n in ("x", "topk_weights", "topk_ids"))
+    (q1, s1), (q2, s2) = Q.quantize_mxfp4(d["w13"].to(DEV)), Q.quantize_mxfp4(d["w2"].to(DEV))
+    g = torch.Generator().manual_seed(9)
+    b13, b2 = (torch.randn(E, n, generator=g).mul(0.1).to(DEV) for n in (2 * N, K))
+    layer = torch.nn.Module()
+    for name, t in (("w13_weight", q1), ("w13_weight_scale", s1), ("w2_weight", q2), ("w2_weight_scale", s2),
+                    ("w13_weight_bias", b13), ("w2_weight_bias", b2)):
+        layer.register_parameter(name, torch.nn.Parameter(t, requires_grad=False))
+    cfg = SimpleNamespace(num_experts=E, no_combine=False, activation="silu", apply_router_weight_on_input=on_input,
+                          routed_scaling_factor=rsf, gemm1_alpha=1.702, gemm1_clamp_limit=7.0)
+    out = F.fused_moe_flagos(SimpleNamespace(runner=SimpleNamespace(config=cfg)), layer, SimpleNamespace(
+        hidden_states=x, topk_output=SimpleNamespace(topk_weights=tw, topk_ids=ti))).hidden_states
+    if M == 0:
+        assert out.shape == (0, K)
+        return
+    rd, gi, si = F._standard_topk_to_triton_kernels(tw, ti, E)
+    pc = [SimpleNamespace(weight_scale=s.transpose(1, 2)) for s in (s1, s2)]
+    ref = flaggems_sglang.triton_kernel_fused_experts_with_bias(
+        x, q1.transpose(1, 2), pc[0], b13, q2.transpose(1, 2), pc[1], b2, rd, gi, si,
+        apply_router_weight_on_input=on_input, gemm1_alpha=1.702, gemm1_clamp_limit=7.0)
+    if rsf is not None:
+        ref.mul_(rsf)
+    assert torch.equal(out, ref)
