@@ -37,7 +37,7 @@ struct GemmParams {
   // fp8 prefill GEMM1: when set, the activation leaves the epilogue already
   // quantized (e4m3 [M*k, N] + fp32 scales [M*k, N/128]) instead of as bf16
   uint8_t* act_q;
-  float* act_qs;
+  float* act_qs;  // (int4 prefill GEMM1: its activation's group sums [M*k, N/128])
   int64_t out_split_stride;  // elements between split partials (GEMM2)
   int n_ntiles;            // output tiles along Nout
   int splits;              // GEMM2 split-K factor (decode path)
@@ -47,11 +47,11 @@ struct GemmParams {
   // GEMM (replaces the dependent routing loads of every workgroup's prologue)
   int4* tile_lut;
   // prefill GEMM2 tail split (0 = off): each XCD's logical tiles run whole
-  // (bf16 rows, y_bf16) except the last partial round's, which are split up
+  // (bf16 rows with y_bf16, else fp32) except the last partial round's, which are split up
   // to tail_split ways along the reduction dim so they fill one round of the
   // XCD's tail_slots workgroup slots; their fp32 partials go to tail_part
   // ([pair][BM][BN], pairs numbered XCD by XCD, tile * S + split within one) and
-  // tail_fold_kernel adds them into the bf16 rows
+  // tail_fold_kernel adds them into the rows
   int tail_split;
   int tail_slots;
   float* tail_part;

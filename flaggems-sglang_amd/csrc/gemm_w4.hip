@@ -1,11 +1,19 @@
-// Prefill grouped GEMM on int4 (W4A16) weights: the nibbles stay 4-bit until
-// they are in registers, so an expert's weights are read once per M-tile at a
-// quarter of their bf16 size.
+// Prefill grouped GEMM on 4-bit weights (int4 W4A16 and MXFP4): the nibbles
+// stay 4-bit until they are in registers, so an expert's weights are read once
+// per M-tile at a quarter of their bf16 size.
 //
-// One ring stage = one quantization group (128 reduction elements): BM x 256
-// bytes of bf16 activations and 256 x 64 bytes of nibbles, with the group's
-// scales, zeros and row sums.  The bf16 number with bits 0x4300 | q is 128 + q
-// (exact), so a stage's MFMAs give t = sum((128 + q) x) per weight row and
+// One ring stage = 128 reduction elements: BM x 256 bytes of bf16 activations
+// and 256 x 64 bytes of nibbles, with their scales (int4: also zeros and row
+// sums).
+//
+// MXFP4: v_cvt_scalef32_pk_bf16_fp4 gives e2m1 x 2^e exactly in bf16, and the
+// MFMAs go straight into the accumulators.  What bounds it (Mixtral M=33 GEMM1,
+// 146 us at first): the scale bytes fetched per stage, a line per lane (110 us
+// without them; now 16 bytes per row and four stages, 122), then the
+// conversions (12 us).
+//
+// int4: the bf16 number with bits 0x4300 | q is 128 + q (exact), so a stage's
+// MFMAs give t = sum((128 + q) x) per weight row and
 // slot, and the group is folded in fp32 as
 //   acc += scale * (t - (128 + zero) * xs),   xs = sum(x) over the group:
 // the streaming kernels' arithmetic (no 16-bit rounding of the dequantized
@@ -13,6 +21,13 @@
 // of 8, so the activations come in that order: x through rows_for_int4_kernel
 // (which also sums the groups), the intermediate straight from GEMM1's
 // epilogue (whose 128 activation columns are one group).
+// What bounds int4: the vector unit and the matrix cores in turn.  A wave's
+// stage is 64 MFMAs (1024 cycles) and about 320 vector instructions (nibbles
+// 112, scales 48, fold 128) of 4 cycles each, and the two waves of a SIMD hardly
+// overlap one's MFMAs with the other's vector work.  Mixtral M=500 GEMM1 390
+// us; without the fold's multiplications 330, without the unpacking as well
+// 307, without the DMA too 267.  The streaming kernels, which read the weights
+// again for every 32 slots: 434-498 us (call 720 -> 600 us, M=800 1152 -> 754).
 #include <algorithm>
 #include <type_traits>
 

@@ -1,0 +1,37 @@
+"""Tile heights that the library picks at both sides of each line (host only)."""
+
+import pytest
+
+from flaggems_sglang import _lib
+
+
+def _bm(wt, M, k, E, K=2048, N=4096, path=0):
+    return _lib.lib().fmoe_fused_block_m(wt, M, k, E, path, K, N)
+
+
+@pytest.mark.parametrize("M,bm", [(1, 16), (80, 16), (81, 32), (183, 32), (184, 64), (391, 64), (392, 128),
+                                  (2047, 160), (2048, 256)])
+def test_bf16_by_mean(M, bm):
+    assert _bm(_lib.W_BF16, M, 1, 8) == bm
+
+
+@pytest.mark.parametrize("M,bm", [(24, 16), (25, 64), (319, 64), (320, 128)])
+def test_fp8_by_mean(M, bm):
+    assert _bm(_lib.W_FP8, M, 1, 8) == bm
+
+
+@pytest.mark.parametrize("wt,N,stream", [(_lib.W_MXFP4, 7168, 1), (_lib.W_MXFP4_TILED, 7168, 3),
+                                         (_lib.W_MXFP4, 7040, 24), (_lib.W_MXFP4_TILED, 7040, 36)])
+def test_mxfp4_by_width_and_layout(wt, N, stream):
+    assert _bm(wt, 8 * stream, 1, 8, N=N) == 16
+    nxt = 32 if stream < 22 else (64 if stream < 48 else 128)
+    assert _bm(wt, 8 * (stream + 1), 1, 8, N=N) == nxt
+    assert _bm(wt, 8 * 49, 1, 8, N=N) == 128
+    for path in (1, 2):
+        assert _bm(wt, 8 * 49, 1, 8, N=N, path=path) == 16
+    assert _lib.lib().fmoe_choose_block_m(wt, 8 * 49, 1, 8, 0) == 16
+
+
+def test_int4_routing_stays_at_16():
+    for M in (1, 100, 700, 5000):
+        assert _bm(_lib.W_INT4, M, 2, 8) == 16 and _bm(_lib.W_INT4_TILED, M, 2, 8) == 16
