@@ -460,6 +460,19 @@ int check_fused(const fmoe_fused_args* a) {
   return FMOE_OK;
 }
 
+// The device pointers of a call with tokens.  Every route passes here: the
+// one-launch, tiny-batch, unpacking and dequantizing ones launch kernels without
+// the stage entry points' own checks.
+int check_pointers(const fmoe_fused_args* a) {
+  if (!a->x || !a->w13 || !a->w2 || !a->topk_ids || !a->topk_weights || !a->out)
+    return fail(FMOE_ERR_INVALID, "fused_experts: null pointer");
+  if (a->wtype != FMOE_W_BF16 && (!a->w13_scale || !a->w2_scale))
+    return fail(FMOE_ERR_INVALID, "fused_experts: these weights need w13_scale and w2_scale");
+  if (is_int4(a->wtype) && (!a->w13_zero || !a->w2_zero))
+    return fail(FMOE_ERR_INVALID, "fused_experts: int4 needs w13_zero and w2_zero");
+  return FMOE_OK;
+}
+
 // Tiled int4 decode of the smallest batches runs as one launch per call
 // (fused_int4_kernel: GEMM1, activation and GEMM2 of a 128-column slice of
 // the intermediate per workgroup) plus the plane sum.  Its N / 128 fp32
@@ -699,8 +712,7 @@ extern "C" size_t fmoe_fused_experts_workspace_bytes(const fmoe_fused_args* a) {
 extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
   if (int st = check_fused(a)) return st;
   if (a->M == 0) return FMOE_OK;
-  if (!a->x || !a->w13 || !a->w2 || !a->topk_ids || !a->topk_weights || !a->out)
-    return fail(FMOE_ERR_INVALID, "fused_experts: null pointer");
+  if (int st = check_pointers(a)) return st;
   if (dequant_prefill(a)) {
     const size_t need = fmoe_fused_experts_workspace_bytes(a);
     if (!a->workspace || a->workspace_bytes < need)

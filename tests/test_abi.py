@@ -85,3 +85,26 @@ def test_argument_errors_map_to_reference_convention():
     assert b"SWIGLU" in L.fmoe_last_error()
     fa.activation = _lib.ACT_SILU
     assert L.fmoe_fused_experts_workspace_bytes(ctypes.byref(fa)) > 0
+
+
+@pytest.mark.parametrize("M", [1, 16, 100, 700, 1100])  # one launch, streaming, unpacking, bf16 copies
+@pytest.mark.parametrize("wt,fields", [
+    (_lib.W_FP8, ("w13_scale", "w2_scale")),
+    (_lib.W_MXFP4, ("w13_scale", "w2_scale")), (_lib.W_MXFP4_TILED, ("w13_scale", "w2_scale")),
+    (_lib.W_INT4, ("w13_scale", "w2_scale", "w13_zero", "w2_zero")),
+    (_lib.W_INT4_TILED, ("w13_scale", "w2_scale", "w13_zero", "w2_zero"))])
+def test_null_scales_and_zeros_are_refused(wt, fields, M):
+    """Every route of the whole-path call, before anything is launched: the
+    other pointers are host memory, which no kernel may see."""
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(64)
+    host = ctypes.addressof(buf)
+    for missing in fields:
+        a = _lib.FusedArgs()
+        a.wtype, a.M, a.K, a.N, a.E, a.top_k, a.group_size = wt, M, 256, 256, 8, 2, 128
+        a.x = a.w13 = a.w2 = a.topk_weights = a.topk_ids = a.out = host
+        for f in fields:
+            setattr(a, f, None if f == missing else host)
+        # no workspace: a library without the check stops there, short of a launch
+        assert L.fmoe_fused_experts(ctypes.byref(a), None) == _lib.FMOE_ERR_INVALID, missing
+        assert b"need" in L.fmoe_last_error()
