@@ -256,7 +256,7 @@ def stage_times(p, reps=10):
     L = _lib.lib()
     M, K, N, E, k = p["M"], p["K"], p["N"], p["E"], p["k"]
     wt = _wt_codes()[p["wtype"]]
-    bm = L.fmoe_choose_block_m(wt, M, k, E, 0)
+    bm = L.fmoe_fused_block_m(wt, M, k, E, 0, K, N)
     kw = p["kw"]
     s13, s2 = kw.get("w1_scale"), kw.get("w2_scale")
     z13, z2 = kw.get("w1_zp"), kw.get("w2_zp")
@@ -420,9 +420,9 @@ def measure(name, steps, warmup, stages=True):
 
     p = make_problem(name)
     wt = _wt_codes()[p["wtype"]]
-    decode = _lib.lib().fmoe_choose_block_m(wt, p["M"], p["k"], p["E"], 0) == 16
+    bm = _lib.lib().fmoe_fused_block_m(wt, p["M"], p["k"], p["E"], 0, p["K"], p["N"])
     timing = "wall clock per call, synchronous launches"
-    if decode:
+    if bm == 16:
         for _ in range(warmup):
             run_op(p)
         t, n_layers = time_op_graph(p, steps)
@@ -432,7 +432,7 @@ def measure(name, steps, warmup, stages=True):
     if stages:
         stages = stage_times(p)
     else:  # profiling the fused path alone: no staged-path launches in the trace
-        stages = {"block_m": _lib.lib().fmoe_choose_block_m(wt, p["M"], p["k"], p["E"], 0)}
+        stages = {"block_m": bm}
     f = flops(p)
     hit, wbytes = weight_bytes_touched(p)
     io_bytes = p["M"] * p["K"] * (2 if p["wtype"] != "fp8" else 1) + p["M"] * p["K"] * 2

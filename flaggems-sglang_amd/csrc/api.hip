@@ -119,6 +119,12 @@ GemmParams base_params(const fmoe_routing* r) {
 // M=40 (10) 497 / 506 and M=64 (16) 613 / 496; fp8 DSV3 M=64 (2 slots) 1724 / 1696, M=128 (4) 1950 / 1836, M=512 (16)
 // 2907 / 1945, K 2048 N 768 E 128 M=32 (2) 132 / 136 and M=64 (4) 157 / 148.
 constexpr int kDecodeMeanBf16 = 10, kDecodeMeanFp8 = 3;
+// Reductions that the fp8 prefill kernels hold the weight scales of; the
+// streaming kernels have no such limit.  A height chosen without the layer's
+// sizes (fmoe_choose_block_m), and a layer above the limit, stream up to
+// kDecodeMeanFp8Any slots per expert.
+constexpr int64_t kFp8PrefillRed = 16384;
+constexpr int kDecodeMeanFp8Any = 16;
 // The streaming kernels keep GEMM2's slot rows in fp32, the prefill kernels
 // of larger batches in bf16: up to this mean the rows are fp32 on both.
 constexpr int kFp32RowsMean = 16;
@@ -136,11 +142,10 @@ bool mean_at_most(int64_t slots, int64_t E, int mean) {
 // (mean 48, bf16: M=400 334 us against 338 with 128 rows, M=512 (64) 385 / 348)
 // or to mean 39 (fp8); bf16 256-row tiles once experts average >= 256 slots,
 // otherwise 128, or 160 as below.
-int choose_block_m(int wtype, int64_t M, int k, int E, int path) {
+int choose_block_m(int wtype, int64_t M, int k, int E, int path, int mean_fp8) {
   const int64_t slots = M * k;
   if (decode_only(wtype) || path == 2) return kDecodeBM;
-  if (path != 1 && mean_at_most(slots, E, wtype == FMOE_W_FP8 ? kDecodeMeanFp8 : kDecodeMeanBf16))
-    return kDecodeBM;
+  if (path != 1 && mean_at_most(slots, E, wtype == FMOE_W_FP8 ? mean_fp8 : kDecodeMeanBf16)) return kDecodeBM;
   const int64_t mean = slots / E;
   if (wtype == FMOE_W_BF16) {
     if (mean >= 256) return 256;
@@ -182,14 +187,15 @@ int mx_block_m(int wtype, int64_t M, int k, int E, int64_t N) {
 // tiles.
 int layer_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {
   if (is_mx(wtype) && path == 0) return mx_block_m(wtype, M, k, E, N);
-  const int bm = choose_block_m(wtype, M, k, E, path);
+  const bool prefill = K <= kFp8PrefillRed && N <= kFp8PrefillRed;
+  const int bm = choose_block_m(wtype, M, k, E, path, prefill ? kDecodeMeanFp8 : kDecodeMeanFp8Any);
   return wtype == FMOE_W_FP8 && bm == 160 && (K > 8192 || N > 8192) ? 128 : bm;
 }
 
 }  // namespace
 
 extern "C" int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path) {
-  return choose_block_m(wtype, M, k, E, path);
+  return choose_block_m(wtype, M, k, E, path, kDecodeMeanFp8Any);
 }
 
 extern "C" int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {

@@ -35,3 +35,15 @@ def test_mxfp4_by_width_and_layout(wt, N, stream):
 def test_int4_routing_stays_at_16():
     for M in (1, 100, 700, 5000):
         assert _bm(_lib.W_INT4, M, 2, 8) == 16 and _bm(_lib.W_INT4_TILED, M, 2, 8) == 16
+
+
+@pytest.mark.parametrize("K,N", [(6144, 32768), (16512, 2048), (2048, 16512)])
+def test_fp8_layers_above_the_staged_scales_stream(K, N):
+    """The prefill kernels hold the scales of reductions up to 16384; larger
+    layers stream up to 16 slots per expert, as the size-free choice does."""
+    for M in (1, 13, 16, 64):
+        assert _bm(_lib.W_FP8, M, 2, 8, K=K, N=N) == 16
+        assert _lib.lib().fmoe_choose_block_m(_lib.W_FP8, M, 2, 8, 0) == 16
+    assert _bm(_lib.W_FP8, 65, 2, 8, K=K, N=N) == 64
+    assert _bm(_lib.W_FP8, 13, 2, 8, K=16384, N=16384) == 64
+    assert _bm(_lib.W_FP8, 12, 2, 8, K=16384, N=16384) == 16

@@ -162,3 +162,14 @@ def test_graph_replays_equal_eager(fmt, M):
         # unrelated eager work between replays
         _ = (torch.randn(1024, 1024, device=DEV) @ torch.randn(1024, 1024, device=DEV)).sum().item()
         assert torch.equal(op(), eager)
+
+
+@pytest.mark.parametrize("K,N", [(128, 16512), (16512, 128)])
+def test_fp8_reductions_above_the_staged_scales(K, N):
+    """A reduction longer than the prefill kernels hold weight scales for, at 4
+    slots per expert: the streaming kernels, whole call and stages."""
+    d = O.make_inputs(16, K, N, 8, 2, wscale=0.02)
+    q1, q2, kw = _weights("fp8", d)
+    out = _run(d, q1, q2, kw)
+    _close(out, _oracle("fp8", d, q1, q2, kw), 5e-2)
+    _close(_staged_fp8(d, q1, q2, kw), _oracle("fp8", d, q1, q2, kw), 5e-2)
