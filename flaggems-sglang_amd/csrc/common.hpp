@@ -44,16 +44,6 @@ __device__ __forceinline__ void round_bf16x2(float& a, float& b) {
   b = __uint_as_float(w & 0xffff0000u);
 }
 
-// n / d for d >= 1 (the sigmoid denominators): reciprocal, one residual step,
-// and the hardware's fix-up for infinities and NaN.  The general division's
-// operand scaling guards denormal operands and quotients that this
-// denominator does not have, at twice the instructions (11 against 5).
-__device__ __forceinline__ float div_ge1(float n, float d) {
-  const float r = __builtin_amdgcn_rcpf(d);
-  const float q = n * r;
-  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, n), r, q), d, n);
-}
-
 // v / s correctly rounded (as a plain division, s > 0), then clamped to the
 // e4m3 range: v * (1/s) plus one FMA-residual correction (inv = 1/s, itself
 // correctly rounded), which restores the rounding the reciprocal product alone
@@ -77,8 +67,11 @@ __device__ __forceinline__ uint32_t pack_e4m3x4(float a, float b, float c, float
 }
 
 __device__ __forceinline__ float silu_mul(float g, float u) {
-  // ops/fused_moe.py:46 — gate / (1 + exp(-gate)) * up, in fp32
-  return div_ge1(g, 1.0f + __expf(-g)) * u;
+  // ops/fused_moe.py:46 — gate / (1 + exp(-gate)) * up, in fp32.  The full
+  // division: a reciprocal with one residual step misses the last bit of one
+  // quotient in 500, and above 2^126 (gates of -87.3 to -88.7) v_rcp_f32
+  // flushes the denormal reciprocal and the quotient with it.
+  return (g / (1.0f + __expf(-g))) * u;
 }
 
 // ------------------------------------------------------------- wave utils

@@ -96,7 +96,7 @@ __device__ __forceinline__ float gemm1_act(const GemmParams& p, float ga, float 
       gv = fminf(gv, p.limit);
       lv = fminf(fmaxf(lv, -p.limit), p.limit);
     }
-    return div_ge1(gv, 1.0f + __expf(-p.alpha * gv)) * (lv + 1.0f) * g;
+    return gv / (1.0f + __expf(-p.alpha * gv)) * (lv + 1.0f) * g;
   } else {
     float gv = ga * g, uv = ua * g;
     round_bf16x2(gv, uv);

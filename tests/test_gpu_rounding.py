@@ -57,3 +57,36 @@ def test_silu_quotient_range(M):
     # one bf16 rounding (half an ulp: 2^-8 of the value); __expf's relative error grows with |g| (below
     # 130 * 2^-24 + 2^-22, far under 2^-12); quotients below 1e-35 may flush
     torch.testing.assert_close(out.float().cpu(), ref.expand(M, K), rtol=2.0 ** -8 + 2.0 ** -12, atol=1e-35)
+
+
+@pytest.mark.parametrize("act", ["silu", "swiglu"])
+@pytest.mark.parametrize("M", [16, 406])  # the streaming kernels; 256-row tiles
+def test_small_quotients_survive(act, M):
+    """Gates whose sigmoid denominator lies above 2^126, where its reciprocal is
+    denormal: the quotient (about 1e-37) is a normal number, and a large up
+    value makes it visible in the output."""
+    import ctypes
+
+    K = N = 128
+    g = torch.tensor([-88.5, -88.0, -87.5, -87.0, -86.5, -86.0, -85.0, -80.0]).repeat(-(-M // 8))[:M]
+    x = torch.zeros(M, K)
+    x[:, 0], x[:, 1] = g, 2.0 ** 60
+    w13 = torch.zeros(1, 2 * N, K)
+    gate, up = (slice(0, N), slice(N, None)) if act == "silu" else (slice(0, None, 2), slice(1, None, 2))
+    w13[:, gate, 0], w13[:, up, 1] = 1.0, 2.0 ** 40
+    x, w13, w2 = (t.to(torch.bfloat16).to(DEV) for t in (x, w13, torch.eye(K).view(1, K, N)))
+    out = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+    tw, ids = torch.ones(M, 1, device=DEV), torch.zeros(M, 1, dtype=torch.int32, device=DEV)
+    a = _lib.FusedArgs()
+    a.wtype, a.x, a.M, a.K, a.N, a.E, a.top_k = _lib.W_BF16, x.data_ptr(), M, K, N, 1, 1
+    a.w13, a.w2, a.group_size, a.topk_weights, a.topk_ids = w13.data_ptr(), w2.data_ptr(), 128, tw.data_ptr(), ids.data_ptr()
+    a.routed_scaling_factor, a.out, a.alpha = 1.0, out.data_ptr(), 1.0
+    a.activation = _lib.ACT_SILU if act == "silu" else _lib.ACT_SWIGLU
+    n = _lib.lib().fmoe_fused_experts_workspace_bytes(ctypes.byref(a))
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n
+    _lib.check(_lib.lib().fmoe_fused_experts(ctypes.byref(a), _lib.stream_of(x)), "fused_experts")
+    d = g.double().view(-1, 1)
+    ref = (d / (1.0 + torch.exp(-d)) * (2.0 ** 100 + (act == "swiglu"))).float()
+    # the bound of test_silu_quotient_range, without its absolute part
+    torch.testing.assert_close(out.float().cpu(), ref.expand(M, K), rtol=2.0 ** -8 + 2.0 ** -12, atol=0)
