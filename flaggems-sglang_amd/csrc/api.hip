@@ -1,4 +1,5 @@
 // C-ABI entry points of the GEMM stages and the whole fused path.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -134,6 +135,34 @@ bool mean_at_most(int64_t slots, int64_t E, int mean) {
   return slots <= mean * (active > 0 ? active : 1);
 }
 
+// Experts of the rank and of the model (equal without an expert map).  With a
+// map a local expert gets anything from its even share of the slots (slots /
+// global: every rank sees the whole batch) to slots / local (tokens dispatched
+// to the rank that holds their experts), and only the device knows which.
+struct Experts {
+  int local, global;
+};
+Experts experts_of(const fmoe_fused_args* a) {
+  return {a->E, a->expert_map && a->n_global > a->E ? a->n_global : a->E};
+}
+
+// The slots per expert that the tile height is for.  While the largest load
+// fits one tile, that load: taller tiles than the even share needs cost little
+// (their padding), a second M-tile reads the expert's weights again.  Above it,
+// twice the even share, but no less than a quarter of the largest load, in
+// tiles of at least 128 rows (a mean of 49 takes these in every format).  Ranks
+// of eight, us a call at the even share / at the largest load, heights for the
+// even share against these: DSV3 fp8 M=512 305 / 495 against 326 / 379, M=1001
+// 316 / 772 against 321 / 605, M=2048 344 / 1092 against 356 / 1094; the same
+// layer in bf16 M=256 510 / 1963 against 513 / 536, M=1001 533 / 1243 against 534 /
+// 917.  For the largest load throughout: M=1001 334 / 598, bf16 M=2048 617 /
+// 1457 (against 554 / 1667).
+int64_t height_mean(int64_t slots, Experts x) {
+  const double largest = static_cast<double>(slots) / x.local;
+  if (x.global <= x.local || largest + 2.0 * std::sqrt(largest) <= 160.0) return slots / x.local;
+  return std::max<int64_t>(49, slots / std::max(x.local, std::min(x.global / 2, 4 * x.local)));
+}
+
 // Tile height for the fused path: 16 = decode kernels, else the prefill tile,
 // from the mean slots per expert (measured on the BASELINE shapes): bf16
 // 32-row tiles while they hold the mean + 2 sd of a uniform routing's
@@ -142,11 +171,17 @@ bool mean_at_most(int64_t slots, int64_t E, int mean) {
 // (mean 48, bf16: M=400 334 us against 338 with 128 rows, M=512 (64) 385 / 348)
 // or to mean 39 (fp8); bf16 256-row tiles once experts average >= 256 slots,
 // otherwise 128, or 160 as below.
-int choose_block_m(int wtype, int64_t M, int k, int E, int path, int mean_fp8) {
-  const int64_t slots = M * k;
+// With an expert map a batch streams while it may hold at most kStreamMeanMap
+// slots per expert and its even share is below the line: prefill tiles that
+// win at one load lose at the other (DSV3 fp8, a rank of eight, M=40: 222
+// against 206 us streaming at the even share, 279 against 327 at the largest).
+constexpr int kStreamMeanMap = 16;
+int choose_block_m(int wtype, int64_t slots, Experts x, int path, int mean_fp8) {
   if (decode_only(wtype) || path == 2) return kDecodeBM;
-  if (path != 1 && mean_at_most(slots, E, wtype == FMOE_W_FP8 ? mean_fp8 : kDecodeMeanBf16)) return kDecodeBM;
-  const int64_t mean = slots / E;
+  if (path != 1 && mean_at_most(slots, x.global, wtype == FMOE_W_FP8 ? mean_fp8 : kDecodeMeanBf16) &&
+      (x.global == x.local || mean_at_most(slots, x.local, kStreamMeanMap)))
+    return kDecodeBM;
+  const int64_t mean = height_mean(slots, x);
   if (wtype == FMOE_W_BF16) {
     if (mean >= 256) return 256;
     if (mean <= 22) return 32;
@@ -173,33 +208,41 @@ int prefill_bn(int wtype, int bm) { return wtype == FMOE_W_BF16 && bm <= 64 ? 12
 // Mixtral M=4 (1 slot per expert) 165 / 149 (128 / 139), M=16 (4) 238 / 196 (186 /
 // 180), M=64 (16) 368 / 230 (286 / 218); TP-8 (N = 1792) M=64 65 / 77 (55 / 77),
 // M=100 (25) 80 / 78 (68 / 78).
-int mx_block_m(int wtype, int64_t M, int k, int E, int64_t N) {
-  const int64_t slots = M * k, used = slots < E ? slots : E;
+// With an expert map the line is for the even share, so that the prefill kernels
+// win at every load (reference sweep's K and N, a rank of eight, M=32: 37 us
+// streaming, 49 with 64-row tiles).
+int mx_block_m(int wtype, int64_t slots, Experts x, int64_t N) {
+  const int64_t used = slots < x.local ? slots : x.local;
   const bool wide = used * (N / 128) >= 448;
   const int mean_stream = wide ? (is_tiled(wtype) ? 3 : 1) : (is_tiled(wtype) ? 36 : 24);
-  if (mean_at_most(slots, E, mean_stream)) return kDecodeBM;
-  const int64_t mean = slots / E;
+  if (mean_at_most(slots, x.global, mean_stream)) return kDecodeBM;
+  const int64_t mean = height_mean(slots, x);
   return mean <= 22 ? 32 : (mean <= 48 ? 64 : 128);
 }
 
 // The height for a K x N layer.  The 160-row fp8 tile stages the weight scales
 // of at most 64 reduction blocks (K, N <= 8192); larger fp8 layers take 128-row
 // tiles.
-int layer_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {
-  if (is_mx(wtype) && path == 0) return mx_block_m(wtype, M, k, E, N);
+int layer_block_m(int wtype, int64_t slots, Experts x, int path, int64_t K, int64_t N) {
+  if (is_mx(wtype) && path == 0) return mx_block_m(wtype, slots, x, N);
   const bool prefill = K <= kFp8PrefillRed && N <= kFp8PrefillRed;
-  const int bm = choose_block_m(wtype, M, k, E, path, prefill ? kDecodeMeanFp8 : kDecodeMeanFp8Any);
+  const int bm = choose_block_m(wtype, slots, x, path, prefill ? kDecodeMeanFp8 : kDecodeMeanFp8Any);
   return wtype == FMOE_W_FP8 && bm == 160 && (K > 8192 || N > 8192) ? 128 : bm;
 }
 
 }  // namespace
 
 extern "C" int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path) {
-  return choose_block_m(wtype, M, k, E, path, kDecodeMeanFp8Any);
+  return choose_block_m(wtype, M * k, Experts{E, E}, path, kDecodeMeanFp8Any);
 }
 
 extern "C" int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {
-  return layer_block_m(wtype, M, k, E, path, K, N);
+  return layer_block_m(wtype, M * k, Experts{E, E}, path, K, N);
+}
+
+extern "C" int fmoe_fused_block_m_ep(int wtype, int64_t M, int k, int E, int n_global, int path, int64_t K,
+                                     int64_t N) {
+  return layer_block_m(wtype, M * k, Experts{E, n_global > E ? n_global : E}, path, K, N);
 }
 
 extern "C" int fmoe_gemm2_splits(int wtype, int64_t K, int64_t N, const fmoe_routing* r, int path) {
@@ -523,21 +566,18 @@ bool dequant_prefill(const fmoe_fused_args* a) {
 // nibbles in registers (gemm_w4.hip; path 1 keeps asking for the bf16 copies).
 // Mixtral shape, streaming kernels / these in us a call: M=256 (64 slots per
 // expert) 421 / 421, M=500 720 / 600, M=800 1152 / 754; TP-8 M=256 104 / 121,
-// M=600 (150) 154 / 132.
+// M=600 (150) 154 / 132.  (With an expert map the even share counts, as for
+// MXFP4; the bf16 copies above are of the local experts and follow the largest load.)
 constexpr int kW4Mean = 80, kW4BM = 128;
 bool w4_route(const fmoe_fused_args* a) {
   if (!is_int4(a->wtype) || a->activation == FMOE_ACT_SWIGLU || a->b13 || a->path != 0) return false;
-  const int experts = a->expert_map && a->n_global > a->E ? a->n_global : a->E;
-  return !mean_at_most(a->M * a->top_k, experts, kW4Mean) && !dequant_prefill(a);
+  return !mean_at_most(a->M * a->top_k, experts_of(a).global, kW4Mean) && !dequant_prefill(a);
 }
 
 FusedLayout layout(const fmoe_fused_args* a) {
   FusedLayout L{};
   const int64_t slots = a->M * a->top_k;
-  // expert parallel: a local expert's share of the slots follows from the
-  // global expert count (the other ranks' experts take the rest)
-  const int experts = a->expert_map && a->n_global > a->E ? a->n_global : a->E;
-  L.bm = layer_block_m(a->wtype, a->M, a->top_k, experts, a->path, a->K, a->N);
+  L.bm = layer_block_m(a->wtype, slots, experts_of(a), a->path, a->K, a->N);
   L.w4 = w4_route(a);
   if (L.w4) L.bm = kW4BM;
   L.max_tiles = fmoe_max_tiles(slots, a->E);

@@ -177,10 +177,11 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     return a.sorted_token_ids, a.expert_ids, a.num_tokens_post_padded
 
 
-def _block_m(wtype: int, M: int, k: int, E: int, path: int, K: int, N: int) -> int:
-    """The fused path's tile height for a K x N layer (fmoe_fused_block_m: the
-    library's own choice, so stage-path routing always matches it)."""
-    return lib().fmoe_fused_block_m(wtype, M, k, E, path, K, N)
+def _block_m(wtype: int, M: int, k: int, E: int, path: int, K: int, N: int, n_global: int = 0) -> int:
+    """The fused path's tile height for a K x N layer, with an expert map of
+    ``n_global`` entries if that is above E (the library's own choice, so
+    stage-path routing always matches it)."""
+    return lib().fmoe_fused_block_m_ep(wtype, M, k, E, n_global, path, K, N)
 
 
 def _standard_topk_to_triton_kernels(topk_weights, topk_ids, n_expts_tot, block_m: Optional[int] = None):
@@ -632,8 +633,8 @@ def fused_experts(
         # SGLang's no_combine contract: [M, k, K] with slot (t, j) = the
         # expert topk_ids[t, j] (routed_scaling_factor not applied, as in the
         # reference hook, ops/fused_moe.py:399-404)
-        a = _align(topk_weights, topk_ids, E, _block_m(wtype, M, k, E, path, K, N), False,
-                   expert_map=emap)
+        bm = _block_m(wtype, M, k, E, path, K, N, 0 if emap is None else emap.numel())
+        a = _align(topk_weights, topk_ids, E, bm, False, expert_map=emap)
         return _run_stages(x, w1, w2, wtype, w1_scale, w2_scale, w1_zp, w2_zp, M, k, E,
                            a.topk_indx, a.gate_indx, a.gate_scal, a.offs_raw, a.offs_pad, a.tile_map,
                            a.n_tiles, a.block_m, apply_router_weight_on_input, 1.0, combine=False,

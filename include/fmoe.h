@@ -261,10 +261,12 @@ int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path);
 /* The tile height fmoe_fused_experts uses for a layer of hidden size K and
  * intermediate size N: fmoe_choose_block_m with the fp8 160 -> 128 substitution
  * above applied (callers that build their own routing for the stage API use
- * this, so they always agree with the fused path; with an expert map E is the
- * global expert count).  Reference counterpart: the
- * block size triton_kernels' matmul_ogs picks for its routing, ops/fused_moe.py:190. */
+ * this, so they always agree with the fused path).  Reference counterpart: the
+ * block size triton_kernels' matmul_ogs picks for its routing, ops/fused_moe.py:190.
+ * _ep: the same for a call with an expert map of n_global entries, E of them local
+ * (n_global <= E: no map). */
 int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N);
+int fmoe_fused_block_m_ep(int wtype, int64_t M, int k, int E, int n_global, int path, int64_t K, int64_t N);
 
 /* Top-k combine (the scatter + sum inside matmul_ogs, ops/fused_moe.py:208-216,
  * and routed_scaling_factor, :399-404): out[t, :] = bf16(scale *

@@ -47,3 +47,32 @@ def test_fp8_layers_above_the_staged_scales_stream(K, N):
     assert _bm(_lib.W_FP8, 65, 2, 8, K=K, N=N) == 64
     assert _bm(_lib.W_FP8, 13, 2, 8, K=16384, N=16384) == 64
     assert _bm(_lib.W_FP8, 12, 2, 8, K=16384, N=16384) == 16
+
+
+@pytest.mark.parametrize("wt,M,bm", [
+    # 32 of 256 experts, top-8; slots per expert: M / 32 at the even share, M / 4 at the largest load
+    (_lib.W_FP8, 64, 16), (_lib.W_FP8, 65, 64), (_lib.W_FP8, 159, 64), (_lib.W_FP8, 160, 128),
+    (_lib.W_FP8, 512, 160), (_lib.W_FP8, 547, 128), (_lib.W_FP8, 1001, 128), (_lib.W_FP8, 2048, 160),
+    (_lib.W_BF16, 64, 16), (_lib.W_BF16, 65, 32), (_lib.W_BF16, 192, 64), (_lib.W_BF16, 256, 128),
+    (_lib.W_BF16, 546, 160), (_lib.W_BF16, 547, 128), (_lib.W_BF16, 2048, 160), (_lib.W_BF16, 4096, 256),
+    # MXFP4: streaming while the even share is (512 GEMM1 workgroups here: 1 slot)
+    (_lib.W_MXFP4, 32, 16), (_lib.W_MXFP4, 33, 32), (_lib.W_MXFP4, 100, 64), (_lib.W_MXFP4, 200, 128),
+    (_lib.W_MXFP4, 1001, 128)])
+def test_expert_parallel_heights(wt, M, bm):
+    L = _lib.lib()
+    assert L.fmoe_fused_block_m_ep(wt, M, 8, 32, 256, 0, 7168, 2048) == bm
+    assert L.fmoe_fused_block_m_ep(wt, M, 8, 32, 0, 0, 7168, 2048) == L.fmoe_fused_block_m(wt, M, 8, 32, 0, 7168, 2048)
+
+
+@pytest.mark.parametrize("wt", [_lib.W_BF16, _lib.W_FP8, _lib.W_MXFP4, _lib.W_MXFP4_TILED])
+@pytest.mark.parametrize("E,n_global,k", [(32, 256, 8), (4, 256, 8), (16, 128, 8), (4, 8, 2), (1, 64, 4)])
+def test_expert_parallel_never_streams_a_full_load(wt, E, n_global, k):
+    """Tokens dispatched to the rank can fill every choice: whatever the even
+    share is, bf16 and fp8 batches of more than 16 such slots per expert run on
+    prefill tiles, of 128 rows or more once the full load needs two tiles."""
+    for M in range(1, 3000, 7):
+        bm = _lib.lib().fmoe_fused_block_m_ep(wt, M, k, E, n_global, 0, 2048, 2048)
+        if wt in (_lib.W_BF16, _lib.W_FP8):
+            assert M * k <= 16 * min(E, M * k) or bm > 16
+        if bm > 16 and M * k > 160 * E:
+            assert bm >= 128

@@ -173,3 +173,30 @@ def test_fp8_reductions_above_the_staged_scales(K, N):
     out = _run(d, q1, q2, kw)
     _close(out, _oracle("fp8", d, q1, q2, kw), 5e-2)
     _close(_staged_fp8(d, q1, q2, kw), _oracle("fp8", d, q1, q2, kw), 5e-2)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4"])
+@pytest.mark.parametrize("M", [30, 150, 400, 900])  # streaming, one tile per expert, two and more
+@pytest.mark.parametrize("load", ["even share", "all local"])
+def test_expert_map_loads(fmt, M, load):
+    """A rank with 8 of 64 experts, its choices spread over all of them or all on
+    its own: the heights chosen for either load, whole call and per-slot rows,
+    against the streaming kernels."""
+    E, n_global, k = 8, 64, 4
+    d = O.make_inputs(M, 256, 384, E, k, wscale=0.05)
+    q1, q2, kw = _weights(fmt, d)
+    emap = torch.full((n_global,), -1, dtype=torch.int32)
+    emap[torch.arange(E) * 8 + 3] = torch.arange(E, dtype=torch.int32)
+    own = (emap >= 0).nonzero().view(-1)
+    g = torch.Generator().manual_seed(M)
+    ids = torch.rand(M, n_global if load == "even share" else E, generator=g).topk(k, 1).indices
+    d["topk_ids"] = (ids if load == "even share" else own[ids]).to(torch.int32)
+    kw = dict(kw, expert_map=emap.to(DEV), global_num_experts=n_global)
+    out = _run(d, q1, q2, kw)
+    dec = _run(d, q1, q2, kw, path=2)
+    tol = 5e-2 if fmt == "fp8" else 2e-2
+    _close(out, dec.cpu(), tol)
+    rows = _run(d, q1, q2, kw, no_combine=True).float()
+    local = emap[d["topk_ids"].long()] >= 0
+    assert torch.count_nonzero(rows.cpu()[~local]) == 0
+    _close(rows.sum(1), dec.cpu(), tol)
