@@ -574,11 +574,21 @@ bool w4_route(const fmoe_fused_args* a) {
   return !mean_at_most(a->M * a->top_k, experts_of(a).global, kW4Mean) && !dequant_prefill(a);
 }
 
-FusedLayout layout(const fmoe_fused_args* a) {
+// Path 0 calls of at most 16 slots per local expert, or of 4-bit weights below
+// the bf16 copies: the streaming kernels take all of them.
+bool streaming_range(const fmoe_fused_args* a) {
+  return a->path == 0 && (decode_only(a->wtype) || mean_at_most(a->M * a->top_k, a->E, kFp32RowsMean));
+}
+
+// `compact`: the layout for a fixed amount of scratch, where the preferred one
+// does not fit: the streaming kernels wherever they can run (no split parts, no
+// copies of x), and bf16 rows from every unsplit prefill GEMM2.
+FusedLayout layout(const fmoe_fused_args* a, bool compact) {
   FusedLayout L{};
   const int64_t slots = a->M * a->top_k;
-  L.bm = layer_block_m(a->wtype, slots, experts_of(a), a->path, a->K, a->N);
-  L.w4 = w4_route(a);
+  L.bm = compact && streaming_range(a) ? kDecodeBM
+                                       : layer_block_m(a->wtype, slots, experts_of(a), a->path, a->K, a->N);
+  L.w4 = !compact && w4_route(a);
   if (L.w4) L.bm = kW4BM;
   L.max_tiles = fmoe_max_tiles(slots, a->E);
   fmoe_routing r{};
@@ -632,7 +642,8 @@ FusedLayout layout(const fmoe_fused_args* a) {
   L.acts = take(fp8 || L.w4 ? 4 * slots * (a->N / 128) : 0);
   // prefill with one split: bf16 rows (see fused path); otherwise fp32 planes
   // (the int4 prefill kernels' rows are fp32, as the streaming kernels' are)
-  L.y_bf16 = L.bm != kDecodeBM && !L.w4 && !is_mx(a->wtype) && L.splits == 1 && !mean_at_most(slots, a->E, kFp32RowsMean);
+  L.y_bf16 = L.bm != kDecodeBM && !L.w4 && !is_mx(a->wtype) && L.splits == 1 &&
+             (compact || !mean_at_most(slots, a->E, kFp32RowsMean));
   L.y = take((L.y_bf16 ? 2 : 4) * static_cast<size_t>(L.splits) * slots * a->K);
   // prefill: tile table, shared by the two GEMM launches (stream order)
   const int bn = prefill_bn(a->wtype, L.bm);
@@ -727,8 +738,6 @@ int fused_tiny(const fmoe_fused_args* a, const FusedLayout& L, char* ws, hipStre
                       a->out, s);
 }
 
-}  // namespace
-
 // The same call on bf16 copies of the weights placed at the workspace start.
 fmoe_fused_args bf16_args(const fmoe_fused_args* a, void* ws) {
   fmoe_fused_args b = *a;
@@ -746,21 +755,26 @@ fmoe_fused_args bf16_args(const fmoe_fused_args* a, void* ws) {
   return b;
 }
 
-extern "C" size_t fmoe_fused_experts_workspace_bytes(const fmoe_fused_args* a) {
-  if (check_fused(a) != FMOE_OK) return 0;
+size_t workspace_bytes(const fmoe_fused_args* a, bool compact) {
   if (dequant_prefill(a)) {
     const fmoe_fused_args b = bf16_args(a, nullptr);
-    return dequant_bytes(a) + layout(&b).total;
+    return dequant_bytes(a) + layout(&b, compact).total;
   }
-  return layout(a).total;
+  return layout(a, compact).total;
 }
 
-extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
-  if (int st = check_fused(a)) return st;
+}  // namespace
+
+extern "C" size_t fmoe_fused_experts_workspace_bytes(const fmoe_fused_args* a) {
+  return check_fused(a) == FMOE_OK ? workspace_bytes(a, false) : 0;
+}
+
+namespace {
+int run_fused(const fmoe_fused_args* a, bool compact, void* stream) {
   if (a->M == 0) return FMOE_OK;
   if (int st = check_pointers(a)) return st;
   if (dequant_prefill(a)) {
-    const size_t need = fmoe_fused_experts_workspace_bytes(a);
+    const size_t need = workspace_bytes(a, compact);
     if (!a->workspace || a->workspace_bytes < need)
       return fail(FMOE_ERR_WORKSPACE, "fused_experts: workspace %zu < %zu bytes", a->workspace_bytes, need);
     const fmoe_fused_args b = bf16_args(a, a->workspace);
@@ -771,9 +785,9 @@ extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
     if (int st = dequant_4bit(a->wtype, a->w2, a->w2_scale, a->w2_zero, a->E, a->K, a->N,
                               static_cast<uint16_t*>(const_cast<void*>(b.w2)), s))
       return st;
-    return fmoe_fused_experts(&b, stream);
+    return run_fused(&b, compact, stream);
   }
-  const FusedLayout L = layout(a);
+  const FusedLayout L = layout(a, compact);
   if (!a->workspace || a->workspace_bytes < L.total)
     return fail(FMOE_ERR_WORKSPACE, "fused_experts: workspace %zu < %zu bytes", a->workspace_bytes,
                 L.total);
@@ -878,6 +892,13 @@ extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
                       a->K, a->routed_scaling_factor, a->out, stream);
 }
 
+}  // namespace
+
+extern "C" int fmoe_fused_experts(const fmoe_fused_args* a, void* stream) {
+  if (int st = check_fused(a)) return st;
+  return run_fused(a, false, stream);
+}
+
 // ------------------------------------------------ no-allocation entry point
 namespace fmoe {
 // The workspace of fmoe_fused_experts_noalloc: one copy per GPU, in the code
@@ -915,14 +936,8 @@ int scratch_for_current_device(void** out) {
 
 extern "C" int fmoe_fused_experts_noalloc(const fmoe_fused_args* a, void* stream) {
   if (int st = check_fused(a)) return st;
-  size_t need = fmoe_fused_experts_workspace_bytes(a);
-  fmoe_fused_args b = *a;
-  // batches that the streaming kernels would also take: those need less
-  if (need > FMOE_NOALLOC_SCRATCH_BYTES && a->path == 0 &&
-      (w4_route(a) || (is_mx(a->wtype) && !dequant_prefill(a)) || mean_at_most(a->M * a->top_k, a->E, kFp32RowsMean))) {
-    b.path = 2;
-    need = fmoe_fused_experts_workspace_bytes(&b);
-  }
+  const bool compact = workspace_bytes(a, false) > FMOE_NOALLOC_SCRATCH_BYTES;
+  const size_t need = workspace_bytes(a, compact);
   if (need > FMOE_NOALLOC_SCRATCH_BYTES)
     return fail(FMOE_ERR_UNSUPPORTED,
                 "fused_experts_noalloc: this call needs %zu bytes of workspace, above the %zu-byte "
@@ -930,7 +945,8 @@ extern "C" int fmoe_fused_experts_noalloc(const fmoe_fused_args* a, void* stream
                 need, static_cast<size_t>(FMOE_NOALLOC_SCRATCH_BYTES));
   void* ws = nullptr;
   if (int st = scratch_for_current_device(&ws)) return st;
+  fmoe_fused_args b = *a;
   b.workspace = ws;
   b.workspace_bytes = FMOE_NOALLOC_SCRATCH_BYTES;
-  return fmoe_fused_experts(&b, stream);
+  return run_fused(&b, compact, stream);
 }

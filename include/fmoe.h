@@ -326,9 +326,11 @@ int fmoe_fused_experts(const fmoe_fused_args* a, void* stream);
  * The workspace is a library-owned device array of FMOE_NOALLOC_SCRATCH_BYTES
  * per GPU (held until the process ends; a->workspace / workspace_bytes are
  * ignored), looked up once per device with the calling thread's current
- * device, which must be the device of the tensors.  Calls whose workspace
- * query exceeds the maximum fail with FMOE_ERR_UNSUPPORTED (e.g. 4-bit
- * weights on the large-batch dequantize route: pass path = 2).  The kernels
+ * device, which must be the device of the tensors.  Where the workspace query
+ * exceeds the maximum, the call takes a smaller layout: the streaming kernels
+ * (4-bit weights, or up to 16 slots per expert), or bf16 GEMM2 rows.  If that
+ * does not fit either it fails with FMOE_ERR_UNSUPPORTED (e.g. 4-bit weights
+ * on the large-batch dequantize route: pass path = 2).  The kernels
  * need no zeroed scratch.  Every call on one GPU shares that GPU's array:
  * calls that overlap in time on one GPU (different streams, threads) race. */
 #define FMOE_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)

@@ -108,3 +108,24 @@ def test_null_scales_and_zeros_are_refused(wt, fields, M):
         # no workspace: a library without the check stops there, short of a launch
         assert L.fmoe_fused_experts(ctypes.byref(a), None) == _lib.FMOE_ERR_INVALID, missing
         assert b"need" in L.fmoe_last_error()
+
+
+@pytest.mark.parametrize("wt,M,K,N,E,k,path,n_global", [
+    (_lib.W_BF16, 256, 7168, 2048, 32, 8, 0, 256), (_lib.W_BF16, 300, 7168, 2048, 32, 8, 0, 256),
+    (_lib.W_BF16, 320, 7168, 2048, 32, 8, 0, 256),  # a rank of eight
+    (_lib.W_BF16, 300, 7168, 2048, 256, 8, 1, 0), (_lib.W_FP8, 400, 7168, 2048, 256, 8, 1, 0),  # up to 16 slots, path 1
+    (_lib.W_INT4, 250, 7168, 128, 256, 8, 2, 0), (_lib.W_MXFP4, 250, 7168, 256, 32, 8, 0, 0),
+    (_lib.W_FP8, 250, 7168, 2048, 256, 8, 0, 0)])
+def test_noalloc_takes_what_fits_some_layout(wt, M, K, N, E, k, path, n_global):
+    """Calls whose preferred layout is above the library's scratch, or close to
+    it, but whose streaming kernels or bf16 rows fit: not refused for their size
+    (with null pointers they end at the pointer check; without a device before it)."""
+    L = _lib.lib()
+    some = ctypes.create_string_buffer(16)
+    a = _lib.FusedArgs()
+    a.wtype, a.M, a.K, a.N, a.E, a.top_k, a.group_size, a.path = wt, M, K, N, E, k, 128, path
+    if n_global:
+        a.expert_map, a.n_global = ctypes.addressof(some), n_global
+    assert L.fmoe_fused_experts_noalloc(ctypes.byref(a), None) in (_lib.FMOE_ERR_INVALID, _lib.FMOE_ERR_HIP)
+    a.M = 40 * M
+    assert L.fmoe_fused_experts_noalloc(ctypes.byref(a), None) == _lib.FMOE_ERR_UNSUPPORTED

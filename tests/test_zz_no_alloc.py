@@ -116,3 +116,39 @@ def test_noalloc_rejects_oversized():
     rc = L.fmoe_fused_experts_noalloc(ctypes.byref(a), torch.cuda.current_stream().cuda_stream)
     assert rc == _lib.FMOE_ERR_UNSUPPORTED
     assert b"scratch maximum" in L.fmoe_last_error()
+
+
+def test_noalloc_rank_of_eight_and_bf16_rows():
+    """A rank of eight at 300 tokens (prefill tiles, bf16 rows: equal to the
+    allocating call), and a prefill call (path 1) of 16 slots per expert whose
+    fp32 rows are above the scratch: the same rows in bf16 fit."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+
+    def problem(M, K, N, E, n_ids, k):
+        w13, w2 = (torch.randn(E, r, c, device=DEV, generator=g).mul(0.02).to(torch.bfloat16)
+                   for r, c in ((2 * N, K), (K, N)))
+        x = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+        ti = torch.rand(M, n_ids, device=DEV, generator=g).topk(k, 1).indices.to(torch.int32)
+        return x, w13, w2, torch.full((M, k), 1.0 / k, device=DEV), ti
+
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    for (M, K, N, E, k, path, n_global), same in (((300, 7168, 128, 32, 8, 0, 256), True),
+                                                  ((512, 16512, 128, 64, 2, 1, 0), False)):
+        x, w13, w2, tw, ti = problem(M, K, N, E, n_global or E, k)
+        emap = torch.full((n_global,), -1, dtype=torch.int32, device=DEV)
+        if n_global:
+            emap[:E] = torch.arange(E, device=DEV)
+        outs = [torch.empty_like(x) for _ in range(2)]
+        args = [_args(_lib.W_BF16, x, w13, w2, tw, ti, o, path=path) for o in outs]
+        for a in args:
+            if n_global:
+                a.expert_map, a.n_global = emap.data_ptr(), n_global
+        n = L.fmoe_fused_experts_workspace_bytes(ctypes.byref(args[0]))
+        assert (n <= SCRATCH_BYTES) == same
+        ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+        args[0].workspace, args[0].workspace_bytes = ws.data_ptr(), n
+        _lib.check(L.fmoe_fused_experts(ctypes.byref(args[0]), st), "fused_experts")
+        _lib.check(L.fmoe_fused_experts_noalloc(ctypes.byref(args[1]), st), "fused_experts_noalloc")
+        a, b = outs[0].float(), outs[1].float()
+        # k bf16 roundings of rows on top of the output's own
+        assert torch.equal(a, b) if same else float((a - b).norm() / a.norm()) < 2.0 ** -7
