@@ -113,19 +113,41 @@ GemmParams base_params(const fmoe_routing* r) {
 }
 
 // Slots per expert (of the experts that can have any) up to which the
-// streaming kernels run; above it the prefill kernels' LDS ring streams the
-// weights faster than the registers do (more bytes in flight per CU), decode
-// vs prefill kernels in us a call: bf16 Qwen3 M=128 (8 slots) 235 / 232, reference
-// sweep M=64 (8) 279 / 282, M=90 (11) 309 / 288 and M=128 (16) 374 / 294, Mixtral
-// M=40 (10) 497 / 506 and M=64 (16) 613 / 496; fp8 DSV3 M=64 (2 slots) 1724 / 1696, M=128 (4) 1950 / 1836, M=512 (16)
-// 2907 / 1945, K 2048 N 768 E 128 M=32 (2) 132 / 136 and M=64 (4) 157 / 148.
-constexpr int kDecodeMeanBf16 = 10, kDecodeMeanFp8 = 3;
+// streaming kernels run.  Above it the prefill kernels' LDS ring streams the
+// weights faster than the registers do (more bytes in flight per CU); the
+// streaming kernels, of 16-slot tiles, read an expert's weights again from its
+// 17th slot on.  The prefill kernels pay their ring's first fill in every round
+// of workgroups and an unfilled last round, so how early they win follows from
+// the workgroups of the two GEMMs at one tile per expert (g1, g2; bf16 64 act /
+// 128 output columns and two workgroups per CU, fp8 128 / 256 and one).
+// Streaming / prefill in us a call:
+//  bf16, g1 + g2 >= 2048, line 10: reference sweep M=64 (8 slots) 279 / 282, M=88
+//    (11) 298 / 286; Qwen3 M=176 (11) 249 / 247; Mixtral M=40 (10) 497 / 506, M=44
+//    (11) 524 / 488, M=64 (16) 662 / 510.
+//  bf16, fewer, line 13: Mixtral TP-2 11 slots 265 / 276, 14 291 / 279; TP-8 12
+//    87 / 92, 14 106 / 92; K 2048 N 4096 E 16 11 174 / 186, 14 181 / 189, 15 200 / 189.
+//  fp8, g1 + g2 >= 1400 and no reduction under 768, line 3: DSV3 M=64 (2) 1724 /
+//    1696, M=128 (4) 1950 / 1836, M=512 (16) 2907 / 1945; K 7168 N 2048 E 32 4 slots 284 / 267;
+//    Qwen3's shape 4 149 / 144; reference sweep 4 186 / 183; K 4096 N 14336 E 16 4 499 / 514, 8 520 / 514.
+//  fp8, others, line 13: Mixtral's shape 5 slots 270 / 295, 11 295 / 317, 14 348 / 321;
+//    TP-8 13 60 / 73, 14 75 / 73; K 4096 N 2048 E 40 (640 + 640) 4 216 / 244, 8 220 / 245;
+//    K 1024 N 512 E 256 (1024 + 1024) 4 109 / 118, 8 121 / 123.
+//  g1 <= 96, for fp8 g2 <= 96 too, line 16: K 1024 N 512 E 8, 16 slots: bf16 25 /
+//    28, fp8 26 / 33; fp8 K 4096 N 8192 E 4 (256, 64), 15 slots 131 / 149.
+constexpr int64_t kFewWgs = 96;
+constexpr int kStreamMeanMid = 13, kStreamMeanMax = 16;
 // Reductions that the fp8 prefill kernels hold the weight scales of; the
-// streaming kernels have no such limit.  A height chosen without the layer's
-// sizes (fmoe_choose_block_m), and a layer above the limit, stream up to
-// kDecodeMeanFp8Any slots per expert.
+// streaming kernels have no such limit.
 constexpr int64_t kFp8PrefillRed = 16384;
-constexpr int kDecodeMeanFp8Any = 16;
+int stream_mean(int wtype, int64_t used, int64_t K, int64_t N) {
+  const bool fp8 = wtype == FMOE_W_FP8;
+  const int bn = fp8 ? 256 : 128;
+  const int64_t g1 = used * ((N + bn / 2 - 1) / (bn / 2)), g2 = used * ((K + bn - 1) / bn);
+  if (g1 <= kFewWgs) return kStreamMeanMax;
+  if (fp8 && (g2 <= kFewWgs || K > kFp8PrefillRed || N > kFp8PrefillRed)) return kStreamMeanMax;
+  if (fp8) return g1 + g2 >= 1400 && K >= 768 && N >= 768 ? 3 : kStreamMeanMid;
+  return g1 + g2 >= 2048 ? 10 : kStreamMeanMid;
+}
 // The streaming kernels keep GEMM2's slot rows in fp32, the prefill kernels
 // of larger batches in bf16: up to this mean the rows are fp32 on both.
 constexpr int kFp32RowsMean = 16;
@@ -171,15 +193,14 @@ int64_t height_mean(int64_t slots, Experts x) {
 // (mean 48, bf16: M=400 334 us against 338 with 128 rows, M=512 (64) 385 / 348)
 // or to mean 39 (fp8); bf16 256-row tiles once experts average >= 256 slots,
 // otherwise 128, or 160 as below.
-// With an expert map a batch streams while it may hold at most kStreamMeanMap
+// With an expert map a batch streams while it may hold at most kStreamMeanMax
 // slots per expert and its even share is below the line: prefill tiles that
 // win at one load lose at the other (DSV3 fp8, a rank of eight, M=40: 222
 // against 206 us streaming at the even share, 279 against 327 at the largest).
-constexpr int kStreamMeanMap = 16;
-int choose_block_m(int wtype, int64_t slots, Experts x, int path, int mean_fp8) {
+int choose_block_m(int wtype, int64_t slots, Experts x, int path, int line) {
   if (decode_only(wtype) || path == 2) return kDecodeBM;
-  if (path != 1 && mean_at_most(slots, x.global, wtype == FMOE_W_FP8 ? mean_fp8 : kDecodeMeanBf16) &&
-      (x.global == x.local || mean_at_most(slots, x.local, kStreamMeanMap)))
+  if (path != 1 && mean_at_most(slots, x.global, line) &&
+      (x.global == x.local || mean_at_most(slots, x.local, kStreamMeanMax)))
     return kDecodeBM;
   const int64_t mean = height_mean(slots, x);
   if (wtype == FMOE_W_BF16) {
@@ -202,18 +223,26 @@ int prefill_bn(int wtype, int bm) { return wtype == FMOE_W_BF16 && bm <= 64 ? 12
 
 // Tile height of MXFP4 batches (path 0): 16 = the streaming kernels, else the
 // prefill kernels that convert in registers.  These stream 256 weight rows per
-// workgroup, so a layer whose GEMM1 makes fewer workgroups than two per CU
-// keeps the streaming kernels longer; tiled weights, which those read faster,
-// somewhat longer too.  Streaming / prefill in us a call, row-major (tiled):
-// Mixtral M=4 (1 slot per expert) 165 / 149 (128 / 139), M=16 (4) 238 / 196 (186 /
-// 180), M=64 (16) 368 / 230 (286 / 218); TP-8 (N = 1792) M=64 65 / 77 (55 / 77),
-// M=100 (25) 80 / 78 (68 / 78).
+// workgroup, so the fewer workgroups GEMM1 makes (g1 = experts with slots * N /
+// 128), the longer the streaming kernels stay ahead, longer still on tiled
+// weights, which they read faster.  Streaming / prefill in us a call, row-major (tiled):
+//  g1 >= 448, lines 1 (3): Mixtral 1 slot per expert 172 / 162 (133 / 150), 5 242 / 194
+//    (191 / 178); TP-2 (448) 2 slots 121 / 111 (97 / 102), 5 129 / 111 (106 / 102);
+//    reference sweep 2 slots 104 / 101 (91 / 96), 5 133 / 129 (116 / 117).
+//  g1 > 96, lines 24 (36): TP-8 (112) 22 slots 80 / 80 (67 / 79), 26 83 / 79 (70 / 76), 40
+//    113 / 93 (93 / 89); K 2048 N 1024 E 16 (128) 26 slots 63 / 61 (56 / 59), 38 76 / 64 (68 /
+//    61).  TP-4 (224) would cross earlier: 5 slots 77 / 75 (66 / 71), 16 103 / 89 (87 / 86).
+//  g1 <= 96, streaming throughout: K 1024 N 512 E 8 (32) 64 slots 31 / 48 (30 / 48), 200
+//    56 / 58 (51 / 58); K 8192 N 1024 E 8 (64) 32 slots 115 / 132 (96 / 126), 64 186 / 168
+//    (153 / 165).
 // With an expert map the line is for the even share, so that the prefill kernels
 // win at every load (reference sweep's K and N, a rank of eight, M=32: 37 us
 // streaming, 49 with 64-row tiles).
 int mx_block_m(int wtype, int64_t slots, Experts x, int64_t N) {
   const int64_t used = slots < x.local ? slots : x.local;
-  const bool wide = used * (N / 128) >= 448;
+  const int64_t g1 = used * (N / 128);
+  if (g1 <= kFewWgs) return kDecodeBM;
+  const bool wide = g1 >= 448;
   const int mean_stream = wide ? (is_tiled(wtype) ? 3 : 1) : (is_tiled(wtype) ? 36 : 24);
   if (mean_at_most(slots, x.global, mean_stream)) return kDecodeBM;
   const int64_t mean = height_mean(slots, x);
@@ -225,15 +254,14 @@ int mx_block_m(int wtype, int64_t slots, Experts x, int64_t N) {
 // tiles.
 int layer_block_m(int wtype, int64_t slots, Experts x, int path, int64_t K, int64_t N) {
   if (is_mx(wtype) && path == 0) return mx_block_m(wtype, slots, x, N);
-  const bool prefill = K <= kFp8PrefillRed && N <= kFp8PrefillRed;
-  const int bm = choose_block_m(wtype, slots, x, path, prefill ? kDecodeMeanFp8 : kDecodeMeanFp8Any);
+  const int bm = choose_block_m(wtype, slots, x, path, stream_mean(wtype, std::min<int64_t>(slots, x.local), K, N));
   return wtype == FMOE_W_FP8 && bm == 160 && (K > 8192 || N > 8192) ? 128 : bm;
 }
 
 }  // namespace
 
 extern "C" int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path) {
-  return choose_block_m(wtype, M * k, Experts{E, E}, path, kDecodeMeanFp8Any);
+  return choose_block_m(wtype, M * k, Experts{E, E}, path, wtype == FMOE_W_FP8 ? kStreamMeanMax : kStreamMeanMid);
 }
 
 extern "C" int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N) {
@@ -563,21 +591,30 @@ bool dequant_prefill(const fmoe_fused_args* a) {
 }
 
 // int4 batches between the two run on the prefill kernels that unpack the
-// nibbles in registers (gemm_w4.hip; path 1 keeps asking for the bf16 copies).
-// Mixtral shape, streaming kernels / these in us a call: M=256 (64 slots per
-// expert) 421 / 421, M=500 720 / 600, M=800 1152 / 754; TP-8 M=256 104 / 121,
-// M=600 (150) 154 / 132.  (With an expert map the even share counts, as for
-// MXFP4; the bf16 copies above are of the local experts and follow the largest load.)
+// nibbles in registers (gemm_w4.hip; path 1 keeps asking for the bf16 copies),
+// where the layer is large enough for their ring's fills: more than kFewWgs
+// GEMM1 workgroups and at least 2^25 weights in w2.  Streaming / these in us a
+// call, row-major (tiled): Mixtral 64 slots per expert 456 / 440 (424 / 449), 82
+// 533 / 470 (492 / 469), 200 1272 / 763 (1195 / 768); TP-8 64 slots 115 / 124 (105 / 125),
+// 82 139 / 127 (130 / 129), 150 167 / 136 (156 / 138); reference sweep 82 355 / 317
+// (324 / 318); Qwen3's shape 82 291 / 253 (267 / 253), 150 456 / 450 (427 / 446); at
+// the size, K 2048 N 1024 E 16, 82 92 / 89 (85 / 88), 200 131 / 97 (122 / 96); worst
+// K 1024 N 512 E 256 160 374 / 388 (349 / 382).  Below the size: K 512 N 4096 E 8 82 slots 55 / 70 (52 / 69); K 1024 N 512 E 32 110 64 / 67
+// (62 / 67), E 8 110 41 / 59 (40 / 58); g1 = 64: K 8192 N 1024 E 8 82 170 / 179 (161 / 180).
+// (With an expert map the even share counts, as for MXFP4; the bf16 copies
+// above are of the local experts and follow the largest load.)
 constexpr int kW4Mean = 80, kW4BM = 128;
+constexpr int64_t kW4Weights = int64_t(1) << 25;
 bool w4_route(const fmoe_fused_args* a) {
   if (!is_int4(a->wtype) || a->activation == FMOE_ACT_SWIGLU || a->b13 || a->path != 0) return false;
+  if (a->E * (a->N / 128) <= kFewWgs || a->E * a->K * a->N < kW4Weights) return false;
   return !mean_at_most(a->M * a->top_k, experts_of(a).global, kW4Mean) && !dequant_prefill(a);
 }
 
 // Path 0 calls of at most 16 slots per local expert, or of 4-bit weights below
 // the bf16 copies: the streaming kernels take all of them.
 bool streaming_range(const fmoe_fused_args* a) {
-  return a->path == 0 && (decode_only(a->wtype) || mean_at_most(a->M * a->top_k, a->E, kFp32RowsMean));
+  return a->path == 0 && (decode_only(a->wtype) || mean_at_most(a->M * a->top_k, a->E, kStreamMeanMax));
 }
 
 // `compact`: the layout for a fixed amount of scratch, where the preferred one

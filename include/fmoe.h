@@ -250,9 +250,10 @@ int fmoe_gemm2_ex(int wtype, const void* act, const float* act_scale, const void
  * 16 selects the decode (streaming) kernels, 32 / 64 / 128 / 160 / 256 the prefill
  * kernels (32 and 256: bf16 only; 160 with fp8 weights needs K and N <= 8192 -- the
  * caller substitutes 128 above that; fmoe_fused_experts does so itself).
- * A choice without the layer's sizes streams fp8 batches of up to 16 slots per
- * expert, which fits every layer; fmoe_fused_block_m knows K and N and takes the
- * prefill kernels from 4 slots on where they hold the layer (K, N <= 16384).
+ * This choice, without the layer's sizes, streams bf16 batches of up to 13 slots
+ * per expert and fp8 ones of up to 16; fmoe_fused_block_m knows K and N and draws
+ * the line by the workgroups they make (from 4 slots on in large fp8 layers; not
+ * below 17 where the fp8 prefill kernels do not hold the layer, K or N > 16384).
  * path: 0 = choose, 1 = prefill, 2 = decode (4-bit weights always report 16
  * here; MXFP4 routing of 32 / 64 / 128 rows, as fmoe_fused_block_m may choose, runs
  * prefill kernels, the other large-batch routes are inside fmoe_fused_experts). */

@@ -5,7 +5,7 @@ import pytest
 from flaggems_sglang import _lib
 
 
-def _bm(wt, M, k, E, K=2048, N=4096, path=0):
+def _bm(wt, M, k, E, K=8192, N=16384, path=0):
     return _lib.lib().fmoe_fused_block_m(wt, M, k, E, path, K, N)
 
 
@@ -17,7 +17,31 @@ def test_bf16_by_mean(M, bm):
 
 @pytest.mark.parametrize("M,bm", [(24, 16), (25, 64), (319, 64), (320, 128)])
 def test_fp8_by_mean(M, bm):
-    assert _bm(_lib.W_FP8, M, 1, 8) == bm
+    assert _bm(_lib.W_FP8, 32 * M, 1, 256, K=7168, N=2048) == bm
+
+
+@pytest.mark.parametrize("wt,E,K,N,line", [
+    (_lib.W_BF16, 8, 4096, 14336, 10), (_lib.W_BF16, 8, 4096, 7168, 13), (_lib.W_BF16, 8, 4096, 1792, 13),
+    (_lib.W_BF16, 64, 1280, 3072, 10), (_lib.W_BF16, 128, 2048, 768, 10), (_lib.W_BF16, 8, 2048, 896, 13),
+    (_lib.W_BF16, 8, 2048, 768, 16), (_lib.W_BF16, 8, 8192, 512, 16),
+    (_lib.W_FP8, 256, 7168, 2048, 3), (_lib.W_FP8, 64, 1280, 3072, 3), (_lib.W_FP8, 128, 2048, 768, 3),
+    (_lib.W_FP8, 32, 7168, 2048, 3), (_lib.W_FP8, 256, 1024, 512, 13), (_lib.W_FP8, 40, 4096, 2048, 13),
+    (_lib.W_FP8, 8, 4096, 14336, 13), (_lib.W_FP8, 8, 4096, 1792, 13), (_lib.W_FP8, 4, 4096, 8192, 16),
+    (_lib.W_FP8, 8, 4096, 1536, 16)])
+def test_streaming_line_by_workgroups(wt, E, K, N, line):
+    """The last streaming mean and the first prefill one, by what the layer's
+    prefill tiles would make of the chip."""
+    assert _bm(wt, line * E, 1, E, K=K, N=N) == 16
+    assert _bm(wt, line * E + 1, 1, E, K=K, N=N) in (32, 64)
+    assert _bm(wt, line * E, 1, E, K=K, N=N, path=1) in (32, 64)
+    assert _lib.lib().fmoe_choose_block_m(wt, 13 * E, 1, E, 0) == 16
+
+
+def test_small_4bit_layers_stream():
+    """Up to 96 GEMM1 workgroups of 256 weight rows."""
+    for wt in (_lib.W_MXFP4, _lib.W_MXFP4_TILED):
+        assert _bm(wt, 8 * 200, 1, 8, K=8192, N=1536) == 16
+        assert _bm(wt, 8 * 200, 1, 8, K=8192, N=1664) == 128
 
 
 @pytest.mark.parametrize("wt,N,stream", [(_lib.W_MXFP4, 7168, 1), (_lib.W_MXFP4_TILED, 7168, 3),
