@@ -1,6 +1,7 @@
 // C-ABI entry points of the GEMM stages and the whole fused path.
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <mutex>
 
 #include "gemm.hpp"
@@ -59,6 +60,12 @@ bool is_tiled(int wt) { return wt == FMOE_W_INT4_TILED || wt == FMOE_W_MXFP4_TIL
 WType to_wt(int wt) {
   return wt == FMOE_W_FP8 ? WType::kFp8
                           : (is_int4(wt) ? WType::kInt4 : (is_mx(wt) ? WType::kMxfp4 : WType::kBf16));
+}
+
+bool aligned16(std::initializer_list<const void*> ptrs) {
+  uintptr_t bits = 0;
+  for (const void* p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);
+  return bits % 16 == 0;
 }
 
 int check_routing(const fmoe_routing* r, const char* who) {
@@ -394,6 +401,8 @@ int gemm1_impl(int wtype, const void* x, const float* x_scale, const void* w13,
     return fail(FMOE_ERR_INVALID, "gemm1: int4 needs w13_scale and w13_zero");
   if (is_mx(wtype) && !w13_scale)
     return fail(FMOE_ERR_INVALID, "gemm1: mxfp4 needs w13_scale (e8m0 block scales)");
+  if (is_mx(wtype) && !is_decode(r) && !aligned16({x, w13, w13_scale}))
+    return fail(FMOE_ERR_INVALID, "gemm1: mxfp4 with block_m > 16 needs 16-byte aligned x, w13 and w13_scale");
   if (is_int4(wtype) && !is_decode(r))
     return fail(FMOE_ERR_UNSUPPORTED, "gemm1: int4 weights need block_m=16 routing");
   if ((path == 1 && is_decode(r)) || (path == 2 && !is_decode(r)))
@@ -466,6 +475,8 @@ int gemm2_impl(int wtype, const void* act, const float* act_scale, const void* w
     return fail(FMOE_ERR_INVALID, "gemm2: int4 needs w2_scale and w2_zero");
   if (is_mx(wtype) && !w2_scale)
     return fail(FMOE_ERR_INVALID, "gemm2: mxfp4 needs w2_scale (e8m0 block scales)");
+  if (is_mx(wtype) && !is_decode(r) && !aligned16({act, w2, w2_scale}))
+    return fail(FMOE_ERR_INVALID, "gemm2: mxfp4 with block_m > 16 needs 16-byte aligned act, w2 and w2_scale");
   if (is_int4(wtype) && !is_decode(r))
     return fail(FMOE_ERR_UNSUPPORTED, "gemm2: int4 weights need block_m=16 routing");
   if ((path == 1 && is_decode(r)) || (path == 2 && !is_decode(r)))
@@ -617,15 +628,27 @@ bool streaming_range(const fmoe_fused_args* a) {
   return a->path == 0 && (decode_only(a->wtype) || mean_at_most(a->M * a->top_k, a->E, kStreamMeanMax));
 }
 
+// Whether the prefill kernels' LDS DMA can fetch the operands: it moves 16-byte
+// pieces (int4 scales and zeros: 4-byte ones), where the streaming kernels
+// load registers, and MXFP4 scales byte by byte, at any address.
+bool dma_aligned(const fmoe_fused_args* a) {
+  if (!aligned16({a->w13, a->w2})) return false;
+  if (is_int4(a->wtype))
+    return ((reinterpret_cast<uintptr_t>(a->w13_scale) | reinterpret_cast<uintptr_t>(a->w2_scale) |
+             reinterpret_cast<uintptr_t>(a->w13_zero) | reinterpret_cast<uintptr_t>(a->w2_zero)) & 3) == 0;
+  if (is_mx(a->wtype)) return aligned16({a->x, a->w13_scale, a->w2_scale});
+  return a->wtype == FMOE_W_FP8 || aligned16({a->x});
+}
+
 // `compact`: the layout for a fixed amount of scratch, where the preferred one
 // does not fit: the streaming kernels wherever they can run (no split parts, no
 // copies of x), and bf16 rows from every unsplit prefill GEMM2.
 FusedLayout layout(const fmoe_fused_args* a, bool compact) {
   FusedLayout L{};
   const int64_t slots = a->M * a->top_k;
-  L.bm = compact && streaming_range(a) ? kDecodeBM
-                                       : layer_block_m(a->wtype, slots, experts_of(a), a->path, a->K, a->N);
-  L.w4 = !compact && w4_route(a);
+  const bool stream = streaming_range(a) && (compact || !dma_aligned(a));
+  L.bm = stream ? kDecodeBM : layer_block_m(a->wtype, slots, experts_of(a), a->path, a->K, a->N);
+  L.w4 = !stream && w4_route(a);
   if (L.w4) L.bm = kW4BM;
   L.max_tiles = fmoe_max_tiles(slots, a->E);
   fmoe_routing r{};
@@ -803,7 +826,15 @@ size_t workspace_bytes(const fmoe_fused_args* a, bool compact) {
 }  // namespace
 
 extern "C" size_t fmoe_fused_experts_workspace_bytes(const fmoe_fused_args* a) {
-  return check_fused(a) == FMOE_OK ? workspace_bytes(a, false) : 0;
+  if (check_fused(a) != FMOE_OK) return 0;
+  size_t bytes = workspace_bytes(a, false);
+  if (streaming_range(a) && (!a->x || !a->w13 || !a->w2)) {
+    // sizes only: operands that turn out unaligned will stream
+    fmoe_fused_args b = *a;
+    b.path = 2;
+    bytes = std::max(bytes, workspace_bytes(&b, false));
+  }
+  return bytes;
 }
 
 namespace {

@@ -184,6 +184,13 @@ def _block_m(wtype: int, M: int, k: int, E: int, path: int, K: int, N: int, n_gl
     return lib().fmoe_fused_block_m_ep(wtype, M, k, E, n_global, path, K, N)
 
 
+def _stage_path(wtype: int, path: int, *operands) -> int:
+    """``path``, or 2 (the streaming kernels) for MXFP4 operands that do not start
+    at a multiple of 16 bytes, which the prefill kernels' DMA needs."""
+    mx = wtype in (W_MXFP4, W_MXFP4_TILED)
+    return 2 if path == 0 and mx and any(t.data_ptr() % 16 for t in operands) else path
+
+
 def _standard_topk_to_triton_kernels(topk_weights, topk_ids, n_expts_tot, block_m: Optional[int] = None):
     """Convert standard top-k output to routing data (ops/fused_moe.py:103-130).
 
@@ -489,7 +496,8 @@ def triton_kernel_fused_experts_with_bias(
     x, w13, w2t, wtype, s13, s2t = _bias_operands(hidden_states, w1, w1_pcg, b1, w2, w2_pcg, b2, E, activation)
     M, Kh = x.shape
     k = routing_data.n_expts_act
-    bm = _block_m(wtype, M, k, E, 0, Kh, w13.shape[1] // 2)
+    path = 0 if s13 is None else _stage_path(wtype, 0, x, w13, w2t, s13, s2t)
+    bm = _block_m(wtype, M, k, E, path, Kh, w13.shape[1] // 2)
     offs_raw, offs_pad, tile_map, n_tiles = _expt_data_for(routing_data, M * k, bm)
     topk_indx = gather_indx.src_indx.to(torch.int32).contiguous()
     gate_indx = gather_indx.dst_indx.to(torch.int32).contiguous()
@@ -633,7 +641,8 @@ def fused_experts(
         # SGLang's no_combine contract: [M, k, K] with slot (t, j) = the
         # expert topk_ids[t, j] (routed_scaling_factor not applied, as in the
         # reference hook, ops/fused_moe.py:399-404)
-        bm = _block_m(wtype, M, k, E, path, K, N, 0 if emap is None else emap.numel())
+        mx_ops = (x, w1, w2, w1_scale, w2_scale) if use_mxfp4_w4a16 else ()
+        bm = _block_m(wtype, M, k, E, _stage_path(wtype, path, *mx_ops), K, N, 0 if emap is None else emap.numel())
         a = _align(topk_weights, topk_ids, E, bm, False, expert_map=emap)
         return _run_stages(x, w1, w2, wtype, w1_scale, w2_scale, w1_zp, w2_zp, M, k, E,
                            a.topk_indx, a.gate_indx, a.gate_scal, a.offs_raw, a.offs_pad, a.tile_map,

@@ -129,3 +129,28 @@ def test_noalloc_takes_what_fits_some_layout(wt, M, K, N, E, k, path, n_global):
     assert L.fmoe_fused_experts_noalloc(ctypes.byref(a), None) in (_lib.FMOE_ERR_INVALID, _lib.FMOE_ERR_HIP)
     a.M = 40 * M
     assert L.fmoe_fused_experts_noalloc(ctypes.byref(a), None) == _lib.FMOE_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("wt,M,fields", [
+    (_lib.W_BF16, 56, ("x", "w13", "w2")), (_lib.W_FP8, 56, ("w13", "w2")),
+    (_lib.W_INT4, 400, ("w13", "w2")), (_lib.W_MXFP4, 400, ("x", "w13", "w2", "w13_scale", "w2_scale"))])
+def test_unaligned_operands_stream(wt, M, fields):
+    """Operands that the prefill kernels' 16-byte DMA cannot fetch take the
+    streaming kernels, as the whole range of those calls once did; a size query
+    without pointers covers both."""
+    L = _lib.lib()
+
+    def size(path=0, **ptrs):
+        a = _lib.FusedArgs()
+        a.wtype, a.M, a.K, a.N, a.E, a.top_k, a.group_size, a.path = wt, M, 4096, 7168, 8, 2, 128, path
+        for f in ("x", "w13", "w2", "w13_scale", "w2_scale", "w13_zero", "w2_zero"):
+            setattr(a, f, ptrs.get(f, ptrs.get("all")))
+        return L.fmoe_fused_experts_workspace_bytes(ctypes.byref(a))
+
+    prefill, stream = size(all=4096), size(path=2, all=4096)
+    assert prefill != stream
+    for f in fields:
+        assert size(all=4096, **{f: 4096 + 8}) == stream
+    assert size() == max(prefill, stream)
+    if wt == _lib.W_INT4:
+        assert size(all=4096, w13_zero=4096 + 4) == prefill and size(all=4096, w2_scale=4096 + 2) == stream

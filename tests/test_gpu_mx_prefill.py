@@ -134,3 +134,36 @@ def test_hook_one_call_equals_stages(M, on_input, rsf):
     if rsf is not None:
         ref.mul_(rsf)
     assert torch.equal(out, ref)
+
+
+def test_unaligned_scales():
+    """Scale bytes that do not start at a multiple of 16 (a view into a larger
+    buffer): the streaming kernels' result, whole call, bias entry and per-slot rows."""
+    from types import SimpleNamespace
+
+    import flaggems_sglang
+
+    d, ids, (q1, s1), (q2, s2) = _problem(COUNTS[32], 512, 7168, seed=6)
+
+    def view(s, off):
+        buf = torch.empty(s.numel() + 16, dtype=torch.uint8, device=DEV)
+        v = buf[off:off + s.numel()].view(s.shape)
+        assert v.data_ptr() % 16 == off
+        return v.copy_(s)
+
+    x, a, b, tw, ti = d["x"].to(DEV), q1.to(DEV), q2.to(DEV), d["topk_weights"].to(DEV), ids.to(DEV)
+    z13, z2 = torch.zeros(8, 2 * 7168, device=DEV), torch.zeros(8, 512, device=DEV)
+
+    def calls(off, path):
+        kw = dict(use_mxfp4_w4a16=True, w1_scale=view(s1, off), w2_scale=view(s2, off), path=path)
+        rd, gi, si = flaggems_sglang.ops.fused_moe._standard_topk_to_triton_kernels(tw, ti, 8)
+        pc = [SimpleNamespace(weight_scale=kw[n].transpose(1, 2)) for n in ("w1_scale", "w2_scale")]
+        bias = flaggems_sglang.triton_kernel_fused_experts_with_bias(
+            x, a.transpose(1, 2), pc[0], z13, b.transpose(1, 2), pc[1], z2, rd, gi, si)
+        return (flaggems_sglang.fused_experts(x, a, b, tw, ti, **kw),
+                flaggems_sglang.fused_experts(x, a, b, tw, ti, no_combine=True, **kw), bias)
+
+    odd, even = calls(1, 0), calls(0, 2)
+    for o, e in zip(odd[:2], even[:2]):
+        assert torch.equal(o, e)
+    assert _rel(odd[2].float().cpu(), calls(0, 0)[2].float().cpu()) < 1e-2
