@@ -61,8 +61,7 @@ def test_heights(bm, K, N):
 
 @pytest.mark.parametrize("bm", sorted(COUNTS))
 def test_bias_swiglu(bm):
-    """The bias entry on routing of each height (narrow layers, so that the
-    routing, not the rule, picks it)."""
+    """The bias entry at each height that the rule picks."""
     import flaggems_sglang
     from types import SimpleNamespace
 
@@ -80,6 +79,30 @@ def test_bias_swiglu(bm):
     ref = O.fused_experts_bias(d["x"], O.mxfp4_dequant(q1, s1), b13, O.mxfp4_dequant(q2, s2), b2,
                                d["topk_weights"], ids, alpha=1.702, limit=7.0).float()
     assert _rel(out, ref) < 1e-2
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("bm,counts", [(32, [17, 1, 32, 2]), (64, [33, 65, 1, 33]), (128, [129, 3, 66, 2])])
+def test_split_inside_a_scale_piece(bm, counts, tiled):
+    """GEMM2 reductions of 20 groups in two parts: the second starts at group 10,
+    inside a 16-byte piece of scale bytes (groups 8 to 11)."""
+    import ctypes
+
+    import flaggems_sglang
+
+    K, N, E = 256, 2560, 24
+    d, ids, (q1, s1), (q2, s2) = _problem(counts * 6, K, N, seed=7)
+    M = ids.shape[0]
+    L, wt = _lib.lib(), _lib.W_MXFP4_TILED if tiled else _lib.W_MXFP4
+    assert L.fmoe_fused_block_m(wt, M, 2, E, 0, K, N) == bm
+    r = _lib.Routing(None, None, None, None, None, None, None, M, 2, E, bm, L.fmoe_max_tiles(2 * M, E))
+    assert L.fmoe_gemm2_splits(wt, K, N, ctypes.byref(r), 0) == 2
+    a, b = q1.to(DEV), q2.to(DEV)
+    if tiled:
+        a, b = Q.tile_mxfp4(a), Q.tile_mxfp4(b)
+    out = flaggems_sglang.fused_experts(d["x"].to(DEV), a, b, d["topk_weights"].to(DEV), ids.to(DEV),
+                                        use_mxfp4_w4a16=True, w1_scale=s1.to(DEV), w2_scale=s2.to(DEV)).float().cpu()
+    assert _rel(out, O.fused_experts_mxfp4(d["x"], q1, s1, q2, s2, d["topk_weights"], ids).float()) < 1e-2
 
 
 def test_scale_bytes_0_and_255():
@@ -102,14 +125,16 @@ def test_scale_bytes_0_and_255():
 @pytest.mark.parametrize("M", [0, 1, 5, 40, 300, 520])
 @pytest.mark.parametrize("on_input,rsf", [(False, None), (True, 2.5)])
 def test_hook_one_call_equals_stages(M, on_input, rsf):
-    """The hook's MXFP4 bias layer (one C call; stages again from 256 slots per
-    expert) against the bias entry on prepared routing: bit-identical."""
+    """The hook's MXFP4 bias layer (one C call up to 255 slots per expert: streaming
+    to M=40, 128-row tiles at M=300; the stages above) against the bias entry on
+    prepared routing, bit-identical, and against the oracle."""
     from types import SimpleNamespace
 
     import flaggems_sglang
     from flaggems_sglang.ops import fused_moe as F
 
-    K, N, E, k = 256, 512, 4, 2
+    K, N, E, k = 256, 3328, 4, 2
+    assert _lib.lib().fmoe_fused_block_m(_lib.W_MXFP4, M, k, E, 0, K, N) == (128 if M >= 300 else 16)
     d = O.make_inputs(max(M, 1), K, N, E, k, wscale=0.05)
     x, tw, ti = (d[n][:M].to(DEV) for n in ("x", "topk_weights", "topk_ids"))
     (q1, s1), (q2, s2) = Q.quantize_mxfp4(d["w13"].to(DEV)), Q.quantize_mxfp4(d["w2"].to(DEV))
@@ -134,6 +159,10 @@ def test_hook_one_call_equals_stages(M, on_input, rsf):
     if rsf is not None:
         ref.mul_(rsf)
     assert torch.equal(out, ref)
+    orc = O.fused_experts_bias(x.cpu(), O.mxfp4_dequant(q1.cpu(), s1.cpu()), b13.cpu(),
+                               O.mxfp4_dequant(q2.cpu(), s2.cpu()), b2.cpu(), tw.cpu(), ti.cpu(), alpha=1.702, limit=7.0,
+                               apply_router_weight_on_input=on_input).float()
+    assert _rel(out.float().cpu(), orc * (1.0 if rsf is None else rsf)) < 1e-2
 
 
 def test_unaligned_scales():

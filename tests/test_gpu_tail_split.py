@@ -1,12 +1,13 @@
 """Prefill GEMM2 tail split on the GPU (fused path).
 
 Calls whose GEMM2 the split rule would cut into fp32 planes (few output tiles,
-a long reduction) run whole tiles as bf16 slot rows and split only each XCD's
-last partial round; ``tail_fold_kernel`` adds the parts.  These shapes take
-that route (asserted through the C ABI's own split rule), with K = 640 so the
-last output tile is partial (640 = 2 x 256 + 128), across the bf16 tile
-heights 64 / 160 / 256, the fp8 128-row tiles and SwiGLU with both biases.  Whole output against the
-oracle, and bit identity across runs.
+a long reduction) run whole tiles as slot rows (bf16, or fp32 up to 16 slots per
+expert) and split only each XCD's last partial round; ``tail_fold_kernel`` adds
+the parts.  These shapes take that route (asserted through the C ABI's own
+split rule), with K = 640 so the last output tile is partial (640 = 2 x 256 +
+128), across the bf16 tile heights 32 (fp32 rows) / 64 / 160 / 256, the fp8
+128-row tiles and SwiGLU with both biases.  Whole output against the oracle,
+and bit identity across runs.
 """
 
 import ctypes
@@ -38,7 +39,7 @@ def _close(out, ref, tol):
     assert rel < tol / 4, f"relative error {rel:.3e}"
 
 
-@pytest.mark.parametrize("M,N,bm", [(64, 8192, 64), (256, 16384, 160), (512, 16384, 256)])
+@pytest.mark.parametrize("M,N,bm", [(30, 8192, 32), (64, 8192, 64), (256, 16384, 160), (512, 16384, 256)])
 def test_bf16_tail_split(M, N, bm):
     K, E, k = 640, 4, 2
     got_bm, tail = _takes_tail_split(_lib.W_BF16, M, K, N, E, k)
@@ -67,7 +68,7 @@ def test_fp8_tail_split():
     _close(a, ref, 5e-2)
 
 
-@pytest.mark.parametrize("M", [64, 256])
+@pytest.mark.parametrize("M", [30, 64, 256])
 def test_bf16_swiglu_bias_tail_split(M):
     """SwiGLU with both biases (alpha, clamp) through the C ABI's fused path at
     tail-split shapes: GEMM2's bias enters the split-0 part only, so every
