@@ -2,7 +2,7 @@
 """Fused-MoE benchmark on one MI355X.
 
 Headline (``value``): Mixtral-8x7B-shape bf16 fused MoE at M=4096 tokens
-(prefill), whole op per step = alignment + GEMM1+SiLU +
+(the headline, prefill), whole op per step = alignment + GEMM1+SiLU +
 GEMM2 + top-k sum, inputs (x, weights, top-k routing) resident in HBM.
 Unit TFLOP/s with FLOPs = 6*M*k*K*N.
 
@@ -15,7 +15,7 @@ Also on the same line:
                 (prefill, % fp8 MFMA peak and % of min(peak, AI*BW)) and
                 Mixtral-shape W4A16 decode at M in {1, 4, 16, 64} (tiled int4
                 weights; M=1 / 16 also row-major), % HBM peak; plus DSV3 at
-                M=1 / 128 and Qwen3 at M=64 / 8192 (the other BASELINE configs).
+                M=1 / 128 and Qwen3 at M=64 / 8192 (the other named workloads).
 
 usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME]
 """
@@ -69,7 +69,7 @@ WORKLOADS = {
 for _m in (1, 4, 17, 64, 1024, 2048, 4096):
     WORKLOADS[f"refsweep_bf16_m{_m}"] = (_m, 1280, 3072, 64, 8, "bf16", "softmax")
 
-# every BASELINE.json point besides the headline, then the reference's sweep
+# every named workload besides the headline, then the reference's sweep
 DEFAULT_SECONDARY = (
     "dsv3_fp8_m4096,dsv3_fp8_m8192,dsv3_fp8_m1,dsv3_fp8_m128,"
     "mixtral_w4a16t_m1,mixtral_w4a16t_m4,mixtral_w4a16t_m16,mixtral_w4a16t_m64,"

@@ -50,10 +50,9 @@ bool valid_wtype(int wt) {
   return wt == FMOE_W_BF16 || wt == FMOE_W_FP8 || wt == FMOE_W_INT4 || wt == FMOE_W_MXFP4 ||
          wt == FMOE_W_INT4_TILED || wt == FMOE_W_MXFP4_TILED;
 }
-// weight formats that only the streaming (decode) kernels read
 bool is_int4(int wt) { return wt == FMOE_W_INT4 || wt == FMOE_W_INT4_TILED; }
 bool is_mx(int wt) { return wt == FMOE_W_MXFP4 || wt == FMOE_W_MXFP4_TILED; }
-bool decode_only(int wt) { return is_int4(wt) || is_mx(wt); }
+bool is_4bit(int wt) { return is_int4(wt) || is_mx(wt); }
 // 4-bit weights in the tiled layout of fmoe_tile_int4
 bool is_tiled(int wt) { return wt == FMOE_W_INT4_TILED || wt == FMOE_W_MXFP4_TILED; }
 
@@ -82,7 +81,8 @@ int check_routing(const fmoe_routing* r, const char* who) {
   return FMOE_OK;
 }
 
-// Decode (block_m 16) or prefill (64 / 128) kernels follow the routing's tile height.
+// Streaming (decode, block_m 16) or prefill kernels (any other height) follow the
+// routing's tile height.
 bool is_decode(const fmoe_routing* r) { return r->block_m == kDecodeBM; }
 
 // Most tiles of height bm that `slots` slots over E experts make: every expert
@@ -193,7 +193,7 @@ int64_t height_mean(int64_t slots, Experts x) {
 }
 
 // Tile height for the fused path: 16 = decode kernels, else the prefill tile,
-// from the mean slots per expert (measured on the BASELINE shapes): bf16
+// from the mean slots per expert (measured on the benchmark's shapes): bf16
 // 32-row tiles while they hold the mean + 2 sd of a uniform routing's
 // per-expert load (mean 22; reference sweep M=128 (mean 16) 294 us against
 // 297 with 64 rows, M=256 (32) 344 / 316); 64-row tiles up to the same bound
@@ -205,7 +205,7 @@ int64_t height_mean(int64_t slots, Experts x) {
 // win at one load lose at the other (DSV3 fp8, a rank of eight, M=40: 222
 // against 206 us streaming at the even share, 279 against 327 at the largest).
 int choose_block_m(int wtype, int64_t slots, Experts x, int path, int line) {
-  if (decode_only(wtype) || path == 2) return kDecodeBM;
+  if (is_4bit(wtype) || path == 2) return kDecodeBM;
   if (path != 1 && mean_at_most(slots, x.global, line) &&
       (x.global == x.local || mean_at_most(slots, x.local, kStreamMeanMax)))
     return kDecodeBM;
@@ -287,7 +287,8 @@ extern "C" int fmoe_gemm2_splits(int wtype, int64_t K, int64_t N, const fmoe_rou
     // Prefill GEMM2 has few output tiles (K / 256 per M-tile): below
     // kPrefillNoSplitWgs tiles, split the reduction dim until the grid covers
     // >= 6 waves of one workgroup per CU, so the last wave's tail stays small.
-    // Partials are summed by moe_sum.
+    // Partials are summed by moe_sum.  (The fused path takes the tail split
+    // instead, of the calls that this rule would split.)
     const int64_t slots = r->n_tokens * r->top_k;
     int64_t tiles = (slots + r->block_m - 1) / r->block_m;
     if (is_mx(wtype)) {
@@ -302,14 +303,13 @@ extern "C" int fmoe_gemm2_splits(int wtype, int64_t K, int64_t N, const fmoe_rou
     }
     const int64_t wgs = tiles * ((K + kPrefillBN - 1) / kPrefillBN);
     if (wgs >= kPrefillNoSplitWgs) return 1;
-    const int64_t stage_elems = wtype == FMOE_W_BF16 ? 32 : 128;
     int64_t sp = (kPrefillTargetWgs + wgs - 1) / (wgs > 0 ? wgs : 1);
-    // each split keeps >= 64 stages: a short reduction gains less from the
-    // split than its extra prologue / epilogue and fp32 planes cost (reference
-    // sweep M=1024 / 2048, 48 stages: unsplit 549 -> 504 / 854 -> 738 us;
-    // Mixtral M=4096, 224 stages, keeps its 3 splits)
-    constexpr int64_t kMinStages = 64;
-    const int64_t max_sp = N / stage_elems / kMinStages > 1 ? N / stage_elems / kMinStages : 1;
+    // Each part keeps 2048 elements in bf16 (32 ring stages), 8192 in fp8 (64):
+    // a short reduction gains less from the split than its extra prologue /
+    // epilogue and fp32 planes cost (reference sweep M=1024 / 2048, N 3072: unsplit
+    // 549 -> 504 / 854 -> 738 us; Mixtral M=4096, N 14336, keeps its 3 splits).
+    const int64_t min_part = wtype == FMOE_W_BF16 ? 2048 : 8192;
+    const int64_t max_sp = N / min_part > 1 ? N / min_part : 1;
     if (sp > max_sp) sp = max_sp;
     if (sp > 4) sp = 4;
     return static_cast<int>(sp < 1 ? 1 : sp);
@@ -574,20 +574,20 @@ bool fused_int4_route(const fmoe_fused_args* a, int bm) {
          fused_int4_fits(a->M * a->top_k, a->K);
 }
 
-// Large batches of 4-bit weights: the decode kernels re-read an expert's
-// weights for every 16-slot tile, so once experts average kDequantMinSlots
-// slots the weights are dequantized once to bf16 (in the workspace) and the
-// bf16 prefill kernels run on them.  Measured on the Mixtral shape (tiled
-// int4, decode kernels vs dequantize + bf16 prefill): M=512 (128 slots per
-// expert) 1.16 vs 1.66 ms, M=1024 (256) 2.20 vs 2.13 ms, M=4096 8.4 vs 3.8 ms;
-// MXFP4 M=1024 2.81 vs 2.14 ms.
+// Large batches of 4-bit weights: once experts average kDequantMinSlots slots
+// the weights are dequantized once to bf16 (in the workspace) and the bf16
+// prefill kernels run on them.  The line was measured against the streaming
+// kernels (Mixtral shape, tiled int4: M=512, 128 slots per expert, 1.16 vs 1.66 ms,
+// M=1024 (256) 2.20 vs 2.13 ms, M=4096 8.4 vs 3.8 ms; MXFP4 M=1024 2.81 vs 2.14 ms).
+// The unpacking kernels, which run below it now (int4 M=800 768 us), have not
+// been measured above it.
 constexpr int64_t kDequantMinSlots = 256;
 
 // The bf16 copies live in the caller's workspace for the duration of the
 // call (2 * E * 3 * N * K bytes: 2.8 GB for the Mixtral shape), so the route is
 // taken automatically only while they stay within kDequantMaxBytes; above it
-// (e.g. a DeepSeek-size int4 layer, ~22 GB) the decode kernels run at every M.
-// path = 1 asks for the route regardless of the size.
+// (e.g. a DeepSeek-size int4 layer, ~22 GB) the kernels that unpack in registers
+// take every larger M too.  path = 1 asks for the route regardless of the size.
 constexpr size_t kDequantMaxBytes = size_t(4) << 30;
 
 // bytes of the bf16 copies of w13 and w2
@@ -596,7 +596,7 @@ size_t dequant_bytes(const fmoe_fused_args* a) {
 }
 
 bool dequant_prefill(const fmoe_fused_args* a) {
-  if (!decode_only(a->wtype) || a->path == 2) return false;
+  if (!is_4bit(a->wtype) || a->path == 2) return false;
   if (a->path == 1) return true;
   return a->M * a->top_k >= kDequantMinSlots * a->E && dequant_bytes(a) <= kDequantMaxBytes;
 }
@@ -625,7 +625,7 @@ bool w4_route(const fmoe_fused_args* a) {
 // Path 0 calls of at most 16 slots per local expert, or of 4-bit weights below
 // the bf16 copies: the streaming kernels take all of them.
 bool streaming_range(const fmoe_fused_args* a) {
-  return a->path == 0 && (decode_only(a->wtype) || mean_at_most(a->M * a->top_k, a->E, kStreamMeanMax));
+  return a->path == 0 && (is_4bit(a->wtype) || mean_at_most(a->M * a->top_k, a->E, kStreamMeanMax));
 }
 
 // Whether the prefill kernels' LDS DMA can fetch the operands: it moves 16-byte

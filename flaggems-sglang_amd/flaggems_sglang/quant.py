@@ -1,8 +1,8 @@
 """Weight preparation for the quantized fused-MoE paths (load time, not the
 hot path): fp8-e4m3fn 128x128 block quantization, uint4 group and MXFP4
 quantization into the layouts ``fused_experts`` reads (plain torch, on
-whatever device the weights live), and the tiling of int4 weights for the
-decode kernels (``tile_int4``, a HIP kernel).
+whatever device the weights live), and the tiling of int4 weights into the
+contiguous blocks that the kernels read (``tile_int4``, a HIP kernel).
 """
 
 from __future__ import annotations

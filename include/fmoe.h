@@ -50,7 +50,7 @@ enum fmoe_wtype {
                           dim), bf16 activations: w13 [E, 2N, K/2] u8 + scale [E, 2N, K/32] u8,
                           w2 [E, K, N/2] u8 + scale [E, K, N/32] u8; element 2i in the low
                           nibble; w = e2m1(q) * 2^(s - 127) */
-  FMOE_W_INT4_TILED = 4, /* FMOE_W_INT4 with the weight bytes tiled for the decode kernels
+  FMOE_W_INT4_TILED = 4, /* FMOE_W_INT4 with the weight bytes tiled in 1 KiB blocks
                             (scales and zeros unchanged): w13 [E, 2N/16, K/128, 1024],
                             w2 [E, K/16, N/128, 1024]; see fmoe_tile_int4 */
   FMOE_W_MXFP4_TILED = 5, /* FMOE_W_MXFP4 with the weight bytes tiled the same way
@@ -248,23 +248,22 @@ int fmoe_gemm2_ex(int wtype, const void* act, const float* act_scale, const void
 
 /* Tile height the library pairs with the GEMM kernels for a problem size:
  * 16 selects the decode (streaming) kernels, 32 / 64 / 128 / 160 / 256 the prefill
- * kernels (32 and 256: bf16 only; 160 with fp8 weights needs K and N <= 8192 -- the
- * caller substitutes 128 above that; fmoe_fused_experts does so itself).
+ * kernels (bf16 all of them; fp8 64 / 128 / 160; MXFP4 32 / 64 / 128; 160 with fp8
+ * weights needs K and N <= 8192 -- the caller substitutes 128 above that;
+ * fmoe_fused_experts does so itself).  path: 0 = choose, 1 = prefill, 2 = decode.
  * This choice, without the layer's sizes, streams bf16 batches of up to 13 slots
- * per expert and fp8 ones of up to 16; fmoe_fused_block_m knows K and N and draws
- * the line by the workgroups they make (from 4 slots on in large fp8 layers; not
- * below 17 where the fp8 prefill kernels do not hold the layer, K or N > 16384).
- * path: 0 = choose, 1 = prefill, 2 = decode (4-bit weights always report 16
- * here; MXFP4 routing of 32 / 64 / 128 rows, as fmoe_fused_block_m may choose, runs
- * prefill kernels, the other large-batch routes are inside fmoe_fused_experts). */
+ * per expert and fp8 ones of up to 16, and reports 16 for 4-bit weights. */
 int fmoe_choose_block_m(int wtype, int64_t M, int k, int E, int path);
 
-/* The tile height fmoe_fused_experts uses for a layer of hidden size K and
- * intermediate size N: fmoe_choose_block_m with the fp8 160 -> 128 substitution
- * above applied (callers that build their own routing for the stage API use
- * this, so they always agree with the fused path).  Reference counterpart: the
+/* The same with the layer's hidden size K and intermediate size N, for callers
+ * that build their own routing for the stage API: the height fmoe_fused_experts
+ * uses for bf16 and fp8 weights, and for MXFP4 below its bf16 copies.  Streaming
+ * ends where the layer's prefill tiles fill the chip (from 4 slots per expert on
+ * in large fp8 layers; not below 17 where the fp8 prefill kernels do not hold the
+ * layer, K or N > 16384).  int4 reports 16, the only height its stages take; the
+ * larger int4 tiles are inside fmoe_fused_experts.  Reference counterpart: the
  * block size triton_kernels' matmul_ogs picks for its routing, ops/fused_moe.py:190.
- * _ep: the same for a call with an expert map of n_global entries, E of them local
+ * _ep: for a call with an expert map of n_global entries, E experts being local
  * (n_global <= E: no map). */
 int fmoe_fused_block_m(int wtype, int64_t M, int k, int E, int path, int64_t K, int64_t N);
 int fmoe_fused_block_m_ep(int wtype, int64_t M, int k, int E, int n_global, int path, int64_t K, int64_t N);
@@ -282,11 +281,13 @@ int fmoe_moe_sum(const float* y, int splits, const int32_t* gate_indx, int64_t M
  * conversion (ops/fused_moe.py:103-216, :341-350, :399-404) with
  * SGLang-layout weights (no per-call transpose, cf. :326-327).  `path`:
  * 0 = choose, 1 = prefill (LDS-tiled) kernels, 2 = decode (streaming) kernels.
- * 4-bit weights (int4, MXFP4) run the decode kernels up to an average of 256
- * slots per expert; above it (or with path 1) the call first dequantizes both
- * weight tensors to bf16 inside the workspace (fmoe_fused_experts_workspace_bytes
- * then includes 2 * E * 3 * K * N bytes for them) and runs the bf16 prefill
- * kernels.
+ * 4-bit weights: small batches run the streaming kernels, larger ones prefill
+ * kernels that convert in registers (int4 from 81 slots per expert, MXFP4 from 2 to
+ * 37, both on layers large enough to fill the chip).  From an average of 256 slots
+ * per expert on, while the copies take at most 4 GiB (or with path 1), the call
+ * first dequantizes both weight tensors to bf16 inside the workspace
+ * (fmoe_fused_experts_workspace_bytes then includes 2 * E * 3 * K * N bytes for them)
+ * and runs the bf16 prefill kernels.
  */
 typedef struct fmoe_fused_args {
   int32_t wtype;

@@ -603,7 +603,7 @@ def fused_experts_w4a16(x, w13_q, w13_sc, w13_z, w2_q, w2_sc, w2_z,
 
 # --------------------------------------------------------------------------
 # seeded input generator (reference rule: seed = M+K+N+E+topk,
-# tests/test_fused_moe.py:50-58; layouts / scales from the BASELINE configs)
+# tests/test_fused_moe.py:50-58; layouts / scales from the benchmark workloads)
 # --------------------------------------------------------------------------
 def make_inputs(M, K, N, E, topk, wscale=0.02, seed=None, routing="softmax",
                 expert_bias_std=0.0, n_group=8, topk_group=4, dtype=torch.bfloat16):

@@ -5,7 +5,7 @@ against SGLang live on a GPU), so these are produced by the CPU oracle
 (oracle/fused_moe_oracle.py) on the reference's own input recipe
 (tests/test_fused_moe.py:50-58: x ~ N(0,1), weights N(0,1)*0.1, softmax top-k,
 seed M+K+N+E+topk) at the reference's FUSED_MOE_SHAPES_SMALL
-(tests/accuracy_utils.py:100-102), the BASELINE tiny config, and small
+(tests/accuracy_utils.py:100-102), the tiny config, and small
 fp8 / int4 / activation / bias cases.
 
 To keep the files small, large inputs are not stored: they are regenerated

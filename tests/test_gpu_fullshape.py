@@ -1,4 +1,4 @@
-"""Full BASELINE shapes on the GPU, through the C ABI.
+"""Full benchmark shapes on the GPU, through the C ABI.
 
 Where the CPU oracle finishes in seconds the whole output is compared
 (DeepSeek-V3 fp8 at E=256 for M = 1 and 128 -- the oracle dequantizes only
@@ -128,7 +128,7 @@ def test_qwen3_bf16_m8192_permutation_and_determinism():
     w2 = _gpu_weights(E, K, N, seed=42)
     gen = torch.Generator(device=DEV).manual_seed(43)
     x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
-    # per-expert bias N(0, 0.5) on the logits skews the routing (BASELINE configs[2])
+    # per-expert bias N(0, 0.5) on the logits skews the routing
     logits = torch.randn(M, E, device=DEV, generator=gen) + \
         torch.randn(E, device=DEV, generator=gen)[None, :] * 0.5
     tw, ti = flaggems_sglang.topk_softmax(logits, k)

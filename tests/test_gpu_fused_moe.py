@@ -3,10 +3,10 @@
 Mirrors the reference's accuracy tests (tests/test_fused_moe.py:84-113: every
 FUSED_MOE_SHAPES entry, plus apply_router_weight_on_input on the small
 shapes; inputs per its _make_inputs, seed M+K+N+E+topk) and adds the
-BASELINE configurations (bf16, skewed routing, fp8 block-scale, int4) at
+benchmark configurations (bf16, skewed routing, fp8 block-scale, int4) at
 sizes the oracle finishes in seconds.  Tolerances: bf16 atol=rtol=2e-2;
 fp8 / int4 5e-2 against the dequantize-then-compute oracle -- with the
-absolute term scaled by the output RMS (_close), and on the BASELINE input
+absolute term scaled by the output RMS (_close), and on the benchmark input
 recipes also exactly as written (_close_literal).
 """
 
@@ -62,7 +62,7 @@ def _close(out, ref, tol):
 def _close_literal(out, ref, tol):
     """north_star's tolerance as written: |out - ref| <= tol + tol * |ref|
     elementwise (torch.testing.assert_close(atol=rtol=tol)).  Used on the
-    BASELINE input recipes (weights N(0, 0.02), outputs of RMS ~1), where
+    benchmark input recipes (weights N(0, 0.02), outputs of RMS ~1), where
     one bf16 ulp of the output is well inside tol; the reference's own test
     shapes (weights N(0,1)*0.1, output RMS ~10, where an output ulp alone is
     0.06) take _close."""
@@ -95,7 +95,7 @@ def test_fused_moe_input_gate(shape):
 @pytest.mark.parametrize("topk", [1, 6, 12])
 @pytest.mark.parametrize("M", [1, 3, 300])
 def test_topk_counts(M, topk):
-    """Top-k counts outside the BASELINE set: 1 (switch routing), 6 and 12
+    """Top-k counts outside the benchmark set: 1 (switch routing), 6 and 12
     (the top-k sum's 8-term batches end part-full), one token (GEMM2 and the
     top-k sum in one launch), decode and prefill; bit-identical reruns."""
     K, N, E = 256, 384, 32
@@ -120,7 +120,7 @@ def test_fused_experts_both_paths(M, path):
 
 
 def test_tiny_config():
-    """M=64, K=128, N=256, E=8, top-2 (fp32 oracle; the
+    """The tiny configuration: M=64, K=128, N=256, E=8, top-2 (fp32 oracle; the
     GPU computes in bf16 with fp32 accumulation)."""
     d = O.make_inputs(64, 128, 256, 8, 2, wscale=0.02)
     out = flaggems_sglang.fused_experts(d["x"].to(DEV), d["w13"].to(DEV), d["w2"].to(DEV),
@@ -142,7 +142,7 @@ def test_routed_scaling_and_no_combine():
     _close(per.float().sum(1), base.float().cpu(), 2e-2)
 
 
-# ------------------------------------------------------------ BASELINE configs
+# ------------------------------------------------------------ benchmark configurations
 def _bf16_case(M, K, N, E, k, bias=0.0, seed=None):
     d = O.make_inputs(M, K, N, E, k, wscale=0.02, expert_bias_std=bias, seed=seed)
     out = flaggems_sglang.fused_experts(d["x"].to(DEV), d["w13"].to(DEV), d["w2"].to(DEV),

@@ -55,7 +55,7 @@ def test_grouped_topk(M, bias):
 
 
 ALIGN_CASES = [
-    # (M, E, k, expert_bias_std) -- tiny, reference small shapes, the BASELINE
+    # (M, E, k, expert_bias_std) -- tiny, reference small shapes, the benchmark
     # configs' routing sizes (Qwen3 skewed, DSV3), multi-chunk sizes
     (1, 8, 2, 0.0), (7, 8, 2, 0.0), (33, 16, 4, 0.0), (64, 8, 2, 0.0), (256, 8, 2, 0.0),
     (257, 8, 2, 0.0), (1024, 128, 8, 0.5), (8192, 128, 8, 0.5), (4096, 256, 8, 0.0),
