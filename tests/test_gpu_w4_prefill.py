@@ -31,6 +31,7 @@ def _unpacks(M, K, N, E, k, n_global=0):
     some = ctypes.create_string_buffer(16)
     a = _lib.FusedArgs()
     a.wtype, a.M, a.K, a.N, a.E, a.top_k, a.group_size = _lib.W_INT4, M, K, N, E, k, 128
+    a.x = a.w13 = a.w2 = 4096  # aligned operands (a query without any covers both routes)
     if n_global:
         a.expert_map, a.n_global = ctypes.addressof(some), n_global
     sizes = []
