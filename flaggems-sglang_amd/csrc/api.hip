@@ -186,10 +186,13 @@ Experts experts_of(const fmoe_fused_args* a) {
 // layer in bf16 M=256 510 / 1963 against 513 / 536, M=1001 533 / 1243 against 534 /
 // 917.  For the largest load throughout: M=1001 334 / 598, bf16 M=2048 617 /
 // 1457 (against 554 / 1667).
+int64_t twice_even_mean(int64_t slots, Experts x) {
+  return slots / std::max(x.local, std::min(x.global / 2, 4 * x.local));
+}
 int64_t height_mean(int64_t slots, Experts x) {
   const double largest = static_cast<double>(slots) / x.local;
   if (x.global <= x.local || largest + 2.0 * std::sqrt(largest) <= 160.0) return slots / x.local;
-  return std::max<int64_t>(49, slots / std::max(x.local, std::min(x.global / 2, 4 * x.local)));
+  return std::max<int64_t>(49, twice_even_mean(slots, x));
 }
 
 // Tile height for the fused path: 16 = decode kernels, else the prefill tile,
@@ -242,17 +245,25 @@ int prefill_bn(int wtype, int bm) { return wtype == FMOE_W_BF16 && bm <= 64 ? 12
 //  g1 <= 96, streaming throughout: K 1024 N 512 E 8 (32) 64 slots 31 / 48 (30 / 48), 200
 //    56 / 58 (51 / 58); K 8192 N 1024 E 8 (64) 32 slots 115 / 132 (96 / 126), 64 186 / 168
 //    (153 / 165).
-// With an expert map the line is for the even share, so that the prefill kernels
-// win at every load (reference sweep's K and N, a rank of eight, M=32: 37 us
-// streaming, 49 with 64-row tiles).
+// With an expert map the even share is held against the line, while the
+// largest load makes at most three 16-slot tiles per expert (kStreamMeanMx), and
+// the height is for twice the even share throughout: MXFP4 tiles of 32 and 64
+// rows run two workgroups per CU, so one for the largest load costs more at the
+// even share than a second tile does at the largest.  Ranks of eight, us a call at the
+// even share / at the largest load: K 7168 N 2048 M=256 325 / 409 with heights for the
+// largest load, 214 / 488 with these, M=540 334 / 753 and 233 / 607; reference sweep
+// M=48 (48 at the largest load) 38 / 74 streaming, 48 / 60 with 32 rows, M=128 50 / 156 and 57 / 75.
+constexpr int kStreamMeanMx = 48;
 int mx_block_m(int wtype, int64_t slots, Experts x, int64_t N) {
   const int64_t used = slots < x.local ? slots : x.local;
   const int64_t g1 = used * (N / 128);
   if (g1 <= kFewWgs) return kDecodeBM;
   const bool wide = g1 >= 448;
   const int mean_stream = wide ? (is_tiled(wtype) ? 3 : 1) : (is_tiled(wtype) ? 36 : 24);
-  if (mean_at_most(slots, x.global, mean_stream)) return kDecodeBM;
-  const int64_t mean = height_mean(slots, x);
+  if (mean_at_most(slots, x.global, mean_stream) &&
+      (x.global == x.local || mean_at_most(slots, x.local, kStreamMeanMx)))
+    return kDecodeBM;
+  const int64_t mean = twice_even_mean(slots, x);
   return mean <= 22 ? 32 : (mean <= 48 ? 64 : 128);
 }
 

@@ -120,7 +120,7 @@ int fmoe_grouped_topk(const float* logits, const float* bias, int64_t M, int E, 
  * FMOE_ERR_INVALID is not detectable for out-of-range ids without a device
  * sync, so ids >= E are counted into no expert and their slots are dropped
  * (gate_scal 0, never read by the GEMMs).
- * Requires 1 <= k <= 32, 1 <= E <= 1024, block_m in {16, 32, 64, 128}.
+ * Requires 1 <= k <= 32, 1 <= E <= 1024, block_m in {16, 32, 64, 128, 160, 256}.
  */
 typedef struct fmoe_align_out {
   int32_t* expt_indx;

@@ -79,9 +79,9 @@ def test_fp8_layers_above_the_staged_scales_stream(K, N):
     (_lib.W_FP8, 512, 160), (_lib.W_FP8, 547, 128), (_lib.W_FP8, 1001, 128), (_lib.W_FP8, 2048, 160),
     (_lib.W_BF16, 64, 16), (_lib.W_BF16, 65, 32), (_lib.W_BF16, 192, 64), (_lib.W_BF16, 256, 128),
     (_lib.W_BF16, 546, 160), (_lib.W_BF16, 547, 128), (_lib.W_BF16, 2048, 160), (_lib.W_BF16, 4096, 256),
-    # MXFP4: streaming while the even share is (512 GEMM1 workgroups here: 1 slot)
-    (_lib.W_MXFP4, 32, 16), (_lib.W_MXFP4, 33, 32), (_lib.W_MXFP4, 100, 64), (_lib.W_MXFP4, 200, 128),
-    (_lib.W_MXFP4, 1001, 128)])
+    # MXFP4: streaming while the even share is (512 GEMM1 workgroups here: 1 slot), then M / 16
+    (_lib.W_MXFP4, 32, 16), (_lib.W_MXFP4, 33, 32), (_lib.W_MXFP4, 367, 32), (_lib.W_MXFP4, 368, 64),
+    (_lib.W_MXFP4, 783, 64), (_lib.W_MXFP4, 784, 128)])
 def test_expert_parallel_heights(wt, M, bm):
     L = _lib.lib()
     assert L.fmoe_fused_block_m_ep(wt, M, 8, 32, 256, 0, 7168, 2048) == bm
@@ -92,11 +92,14 @@ def test_expert_parallel_heights(wt, M, bm):
 @pytest.mark.parametrize("E,n_global,k", [(32, 256, 8), (4, 256, 8), (16, 128, 8), (4, 8, 2), (1, 64, 4)])
 def test_expert_parallel_never_streams_a_full_load(wt, E, n_global, k):
     """Tokens dispatched to the rank can fill every choice: whatever the even
-    share is, bf16 and fp8 batches of more than 16 such slots per expert run on
-    prefill tiles, of 128 rows or more once the full load needs two tiles."""
+    share is, batches of more than 16 such slots per expert (MXFP4: 48) run on
+    prefill tiles, bf16 and fp8 ones of 128 rows or more once the full load needs
+    two tiles."""
+    mx = wt in (_lib.W_MXFP4, _lib.W_MXFP4_TILED)
+    N = 12928 // E // 128 * 128 + 128 if mx else 2048  # more than 96 GEMM1 workgroups
     for M in range(1, 3000, 7):
-        bm = _lib.lib().fmoe_fused_block_m_ep(wt, M, k, E, n_global, 0, 2048, 2048)
-        if wt in (_lib.W_BF16, _lib.W_FP8):
-            assert M * k <= 16 * min(E, M * k) or bm > 16
-        if bm > 16 and M * k > 160 * E:
+        bm = _lib.lib().fmoe_fused_block_m_ep(wt, M, k, E, n_global, 0, 2048, N)
+        if M * k > (48 if mx else 16) * min(E, M * k):
+            assert bm > 16
+        if not mx and M * k > 160 * E:
             assert bm >= 128

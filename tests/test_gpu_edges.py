@@ -183,7 +183,7 @@ def test_expert_map_loads(fmt, M, load):
     its own: the heights chosen for either load, whole call and per-slot rows,
     against the streaming kernels."""
     E, n_global, k = 8, 64, 4
-    d = O.make_inputs(M, 256, 384, E, k, wscale=0.05)
+    d = O.make_inputs(M, 256, 1664, E, k, wscale=0.05)
     q1, q2, kw = _weights(fmt, d)
     emap = torch.full((n_global,), -1, dtype=torch.int32)
     emap[torch.arange(E) * 8 + 3] = torch.arange(E, dtype=torch.int32)
